@@ -406,11 +406,27 @@ extern "C" int moe_layer_forward_mx(
     moe::set_error(_moe_fn, "%s", saved);                      \
     return rc;                                                 \
   }
+  // Above 32 rows per expert the MXFP4 experts run the block kernels: their tiles go
+  // into the row-tile list's room (at most R / 128 + E of them, which is no more than the
+  // R / 64 + N row tiles it is sized for, N >= E), their segments (8 bytes each) into the
+  // fp8 block tiles' (24 bytes for each of NB / 256 + E, NB >= R).
+  const bool block = use_block(T, K, E) && mx_block_ok(T, H, I, E, K, wfmt, w13, w13_scale, w2, w2_scale);
+  const int mbt = block ? mx_block_max_tiles(T, K, E) : 0;
   TileOut to{};
   to.tiles = (int4*)w.tiles;
-  to.num_tiles = w.num_tiles;
-  to.max_tiles = max_tiles;
-  to.mt = mt;
+  if (block) {
+    MOE_CHECK_ARG(mbt <= max_tiles && mbt <= 3 * moe_max_block_tiles(T, K, E, N, B, 0),
+                  "tile list of %d block tiles does not fit the workspace", mbt);
+    to.seg = (int2*)w.btiles;
+    to.num_tiles = w.bnum;
+    to.max_tiles = mbt;
+    to.mt = kMxBlockTileRows;
+    to.span = 1;
+  } else {
+    to.num_tiles = w.num_tiles;
+    to.max_tiles = max_tiles;
+    to.mt = mt;
+  }
   to.compact = 1;
   to.row_shared = R;
   // Residual add + RMSNorm: up to a few tokens inside the logits launch, else in a
@@ -434,6 +450,14 @@ extern "C" int moe_layer_forward_mx(
     MOE_STEP(blockwise_mapping(ids, nullptr, nullptr, T, K, E, B, N, w.tpid, w.b2e, w.cond, w.counts,
                                w.inv, nullptr, w.map_ws, w.map_ws_bytes, to, stream));
   if (!fz.quant_done) MOE_STEP(moe_act_quant_mx(xr, T, H, w.xq, xs, stream));
+  if (block) {
+    MOE_STEP(layer_gate_up_mx_block(w.xq, xs, T, H, I, E, w13, w13_scale, b13, w.tpid, w.tiles, w.btiles,
+                                    w.bnum, mbt, act, gate_lo, gate_hi, up_lo, up_hi, w.hq, hs, stream));
+    MOE_STEP(layer_down_mx_block(w.hq, hs, T, H, I, E, w2, w2_scale, b2, w.tiles, w.btiles, w.bnum, mbt,
+                                 R, w.y, stream));
+    MOE_STEP(moe_combine(w.y, w.inv, wts, K, T, H, (int)R, 0, out_bf16, stream));
+    return MOE_OK;
+  }
   MOE_STEP(layer_gate_up_mx(w.xq, xs, T, H, I, E, wfmt, w13, w13_scale, b13, nullptr, nullptr,
                             nullptr, 0, w.tpid, (int)NB, w.tiles, w.num_tiles, max_tiles, mt, act,
                             gate_lo, gate_hi, up_lo, up_hi, w.hq, hs, stream));

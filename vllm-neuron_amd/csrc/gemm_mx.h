@@ -1,0 +1,53 @@
+// Shared by the MX expert GEMM kernels (gemm_mx.hip, gemm_mx_block.hip): the kernel
+// arguments, the scaled MFMA and the activation.
+#pragma once
+
+#include <type_traits>
+
+#include "moe_common.h"
+
+namespace moe {
+
+constexpr int kFmtFp8 = 0;  // MFMA format codes (cbsz / blgp) of the scaled instruction
+constexpr int kFmtFp4 = 4;
+
+struct MxArgs {
+  const uint8_t* a;    // fp8 activations: x [T, H] (gate_up) or h [rows, I] (down)
+  const uint8_t* as;   // their E8M0 scales [rows, K/32]
+  const uint8_t* w;    // routed weights, packed (fp4: K/2 bytes per row; fp8: K)
+  const uint8_t* ws;   // routed weight scales [E, rows_w, K/32]
+  const float* bias;   // routed bias [E, rows_w] (fp32) or null
+  const uint8_t* wsh;  // shared-expert weights / scales / bias
+  const uint8_t* wssh;
+  const float* bsh;
+  const int32_t* tpid;
+  const int4* tiles;  // {expert, first slot, rows, first hq / y row}
+  const int32_t* num_tiles;
+  uint8_t* hq;
+  uint8_t* hs;
+  uint16_t* y;
+  int T, H, I, E, nsh;
+  long NB;
+  int act;  // 0 SiLU, 1 Swish (g * sigmoid(1.702 g))
+  float gate_lo, gate_hi, up_lo, up_hi;
+  // the layer at one token (tiles from its own mapping: one row each, token 0)
+  int one;
+  long rows;  // rows of h (block kernels)
+};
+
+__device__ __forceinline__ v4f mfma_mx(const v8i& a, const v8i& b, const v4f& c, int sa, int sb,
+                                      std::integral_constant<int, kFmtFp8>) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, kFmtFp8, kFmtFp8, 0, sa, 0, sb);
+}
+__device__ __forceinline__ v4f mfma_mx(const v8i& a, const v8i& b, const v4f& c, int sa, int sb,
+                                      std::integral_constant<int, kFmtFp4>) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, kFmtFp8, kFmtFp4, 0, sa, 0, sb);
+}
+
+__device__ __forceinline__ float mx_act(float g, int act) {
+  // hardware reciprocal (about 1 ulp): h only feeds the MXFP8 quantization
+  const float k = act ? -1.702f : -1.0f;
+  return g * __builtin_amdgcn_rcpf(1.0f + __expf(k * g));
+}
+
+}  // namespace moe

@@ -144,6 +144,17 @@ __device__ __forceinline__ void load_lds4(const void* g, uint8_t* lds_wave_base)
   __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)lds_wave_base, 4, 0, 0);
 }
 
+// Direct-to-LDS loads through a buffer descriptor (four scalar registers) with a 32-bit
+// lane offset and a scalar offset: no 64-bit lane address, so a loop over many loads
+// holds one register per distinct lane offset. Reads past `bytes` return 0.
+typedef __amdgpu_buffer_rsrc_t buf_rsrc_t;
+__device__ __forceinline__ buf_rsrc_t buf_rsrc(const void* p, long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
+}
+__device__ __forceinline__ void buf_lds16(buf_rsrc_t r, uint32_t voff, int soff, uint8_t* lds_wave_base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_wave_base, 16, (int)voff, soff, 0, 0);
+}
+
 // LDS byte address of a pointer into a __shared__ object.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   typedef __attribute__((address_space(3))) const uint8_t* lds_cptr;
