@@ -151,8 +151,9 @@ typedef __amdgpu_buffer_rsrc_t buf_rsrc_t;
 __device__ __forceinline__ buf_rsrc_t buf_rsrc(const void* p, long bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
 }
+template <bool NT = false>  // NT: the non-temporal hint, as load_lds16_nt
 __device__ __forceinline__ void buf_lds16(buf_rsrc_t r, uint32_t voff, int soff, uint8_t* lds_wave_base) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_wave_base, 16, (int)voff, soff, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_wave_base, 16, (int)voff, soff, 0, NT ? 2 : 0);
 }
 
 // LDS byte address of a pointer into a __shared__ object.
