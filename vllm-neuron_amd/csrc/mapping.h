@@ -46,16 +46,47 @@ static inline size_t map_ws_bytes(int T, int E) {
   return 256 + 2 * align256((size_t)nch * E * 4) + 2 * align256((size_t)E * 4);
 }
 
+// Calls f(i, v) for each nonzero v = a[i], i in [0, n), over the threads of the workgroup.
+// 16-byte loads, eight in flight per thread: a row of affinities holds top-k nonzeros
+// among E, so the pass is its loads, and a chunk's rows are read by one workgroup.
+template <class F>
+static __device__ __forceinline__ void for_nonzero(const float* a, int n, const F& f) {
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  int done = 0;
+  if (((uintptr_t)a & 15) == 0) {
+    constexpr int U = 8;
+    const float4* a4 = (const float4*)a;
+    const int n4 = n >> 2;
+    for (int i0 = tid; i0 < n4; i0 += U * nthr) {
+      float4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = a4[min(i0 + u * nthr, n4 - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * nthr;
+        if (i >= n4) continue;
+        if (v[u].x != 0.f) f(4 * i, v[u].x);
+        if (v[u].y != 0.f) f(4 * i + 1, v[u].y);
+        if (v[u].z != 0.f) f(4 * i + 2, v[u].z);
+        if (v[u].w != 0.f) f(4 * i + 3, v[u].w);
+      }
+    }
+    done = n4 << 2;
+  }
+  for (int i = done + tid; i < n; i += nthr)
+    if (a[i] != 0.f) f(i, a[i]);
+}
+
 static __device__ __forceinline__ void build_chunk_mask(uint32_t (*bm)[8], const int32_t* ids,
                                                  const float* aff, int T, int K, int E, int t0,
                                                  int32_t* status) {
   for (int i = threadIdx.x; i < E * 8; i += blockDim.x) bm[i >> 3][i & 7] = 0u;
   __syncthreads();
+  const int rows = min(kChunk, T - t0);
   if (ids != nullptr) {
-    for (int i = threadIdx.x; i < kChunk * K; i += blockDim.x) {
-      int tl = i / K, t = t0 + tl;
-      if (t >= T) break;
-      int e = ids[(size_t)t * K + (i - tl * K)];
+    for (int i = threadIdx.x; i < rows * K; i += blockDim.x) {
+      const int tl = i / K;
+      const int e = ids[(size_t)t0 * K + i];
       if (e >= 0 && e < E) {
         atomicOr(&bm[e][tl >> 5], 1u << (tl & 31));
       } else if (e >= E && status != nullptr) {
@@ -63,12 +94,10 @@ static __device__ __forceinline__ void build_chunk_mask(uint32_t (*bm)[8], const
       }
     }
   } else {
-    for (int i = threadIdx.x; i < kChunk * E; i += blockDim.x) {
-      int tl = i / E, t = t0 + tl;
-      if (t >= T) break;
-      int e = i - tl * E;
-      if (aff[(size_t)t * E + e] != 0.f) atomicOr(&bm[e][tl >> 5], 1u << (tl & 31));
-    }
+    for_nonzero(aff + (size_t)t0 * E, rows * E, [&](int i, float) {
+      const int tl = i / E, e = i - tl * E;
+      atomicOr(&bm[e][tl >> 5], 1u << (tl & 31));
+    });
   }
   __syncthreads();
 }
@@ -119,12 +148,54 @@ static __device__ __forceinline__ int block_inclusive_sum(int v, int* s_wave) {
 static __host__ __device__ inline int block_tiles_cap(int max_tiles) {
   return max(3 * max_tiles / 16, (max_tiles + 7) / 8);
 }
+static __device__ inline int block_tile_cost(int rows) { return 3 + (rows + 63) / 64; }
+// hdr[1..9] from the wanted cuts of XCDs 1..7; one thread.
+static __device__ inline void block_tile_header(const int* want, int n, int max_tiles, int32_t* hdr) {
+  const int cap = block_tiles_cap(max_tiles);  // 8 cap >= max_tiles >= n
+  int prev = 0;
+  hdr[1] = 0;
+  for (int x = 1; x < 8; ++x) {
+    // monotone, at most cap tiles in this range and at most cap in each later one
+    const int v = min(max(want[x], max(prev, n - (8 - x) * cap)), min(prev + cap, n));
+    hdr[1 + x] = v;
+    prev = v;
+  }
+  hdr[9] = n;
+}
+// From the experts, in tile order: expert i (i < nexp) starts at tile first(i) after tiles of
+// cost excl(i), both non-decreasing; total cost C over n tiles. The cut of XCD x is the
+// start whose cost is nearest to x C / 8: seven threads search for it. (Ranking every start
+// against every cut with LDS atomics took 20 us of the mapping's scan launch.)
+template <class FirstF, class ExclF>
+static __device__ void block_tile_cuts_experts(int nexp, const FirstF& first, const ExclF& excl, long C,
+                                               int n, int max_tiles, int32_t* __restrict__ hdr) {
+  __shared__ int s_want[8];
+  const int x = threadIdx.x;
+  if (x >= 1 && x < 8) {
+    int lo = 0, hi = nexp;  // first start past x C / 8
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (8 * (long)excl(mid) <= x * C) lo = mid + 1;
+      else hi = mid;
+    }
+    int w = n;
+    if (lo > 0) {
+      w = first(lo - 1);
+      if (lo < nexp && 8 * (long)excl(lo) - x * C < x * C - 8 * (long)excl(lo - 1)) w = first(lo);
+    }
+    s_want[x] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) block_tile_header(s_want, n, max_tiles, hdr);
+}
+// From the tile list itself (written by this workgroup, stores complete).
 static __device__ void block_tile_cuts(const int4* __restrict__ tiles, int n, int max_tiles,
                                        int32_t* __restrict__ hdr, int* s_wave) {
   __shared__ unsigned long long s_best[8];
+  __shared__ int s_want8[8];
   __shared__ long s_tot;
-  const int tid = threadIdx.x;
-  auto cost = [&](int t) { return 3 + (tiles[t].z + 63) / 64; };
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto cost = [&](int t) { return block_tile_cost(tiles[t].z); };
   if (tid < 8) s_best[tid] = ~0ull;
   int part = 0;
   for (int t = tid; t < n; t += blockDim.x) part += cost(t);
@@ -138,30 +209,27 @@ static __device__ void block_tile_cuts(const int4* __restrict__ tiles, int n, in
     const int c = t < n ? cost(t) : 0;
     const int ci = block_inclusive_sum(c, s_wave);
     const long excl = base + ci - c;
-    if (t < n && (t == 0 || tiles[t].x != tiles[t - 1].x)) {
-      for (int x = 1; x < 8; ++x) {
-        const long d = 8 * excl - (long)x * C;
-        atomicMin(&s_best[x], ((unsigned long long)(d < 0 ? -d : d) << 20) | (unsigned)t);
+    const bool start = t < n && (t == 0 || tiles[t].x != tiles[t - 1].x);
+    // nearest start of the wave for each cut, one atomic per wave and cut
+#pragma unroll
+    for (int x = 1; x < 8; ++x) {
+      const long d = 8 * excl - (long)x * C;
+      unsigned long long v = start ? ((unsigned long long)(d < 0 ? -d : d) << 20) | (unsigned)t : ~0ull;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long w = __shfl_xor(v, o, 64);
+        v = w < v ? w : v;
       }
+      if (lane == 0 && v != ~0ull) atomicMin(&s_best[x], v);
     }
     if (tid == (int)blockDim.x - 1) s_tot = ci;  // the chunk's total
     __syncthreads();
     base += s_tot;
     __syncthreads();
   }
-  if (tid == 0) {
-    const int cap = block_tiles_cap(max_tiles);  // 8 cap >= max_tiles >= n
-    int prev = 0;
-    hdr[1] = 0;
-    for (int x = 1; x < 8; ++x) {
-      int v = s_best[x] == ~0ull ? n : (int)(s_best[x] & 0xFFFFF);
-      // monotone, at most cap tiles in this range and at most cap in each later one
-      v = min(max(v, max(prev, n - (8 - x) * cap)), min(prev + cap, n));
-      hdr[1 + x] = v;
-      prev = v;
-    }
-    hdr[9] = n;
-  }
+  if (tid < 8) s_want8[tid] = s_best[tid] == ~0ull ? n : (int)(s_best[tid] & 0xFFFFF);
+  __syncthreads();
+  if (tid == 0) block_tile_header(s_want8, n, max_tiles, hdr);
 }
 
 // Everything after the per-expert counts: block offsets (exclusive scan of
@@ -309,11 +377,23 @@ static __device__ void finish_mapping(int T, int E, int B, int N, int run, int32
     }
   }
   if (tid == 0) to.num_tiles[0] = min(ntiles + to.n_shared * per, to.max_tiles);
-  if (to.span) {  // block tiles: the XCD ranges (the tile stores above are this workgroup's)
+  if (to.span) {  // block tiles: the XCD ranges, from the experts' costs
+    __shared__ int s_cost[kMapMaxE];  // inclusive
+    int cost = 0;
+    if (tid < E && nt > 0) {
+      const int h = (run + nt - 1) / nt;  // height of all but the last tile
+      cost = (nt - 1) * block_tile_cost(h) + block_tile_cost(run - (nt - 1) * h);
+    }
+    const int ccost = block_inclusive_sum(cost, s_wave);
+    if (tid < E) s_cost[tid] = ccost;
     __syncthreads();
-    __threadfence_block();
-    block_tile_cuts(to.tiles, min(ntiles + to.n_shared * per, to.max_tiles), to.max_tiles,
-                    to.num_tiles, s_wave);
+    const int csh = per > 0 ? (per - 1) * block_tile_cost(hsh) + block_tile_cost(T - (per - 1) * hsh) : 0;
+    const int n = ntiles + to.n_shared * per;
+    block_tile_cuts_experts(
+        E + to.n_shared,
+        [&](int i) { return min(i == 0 ? 0 : i < E ? s_tile[i - 1] : ntiles + (i - E) * per, to.max_tiles); },
+        [&](int i) { return i == 0 ? 0 : i < E ? s_cost[i - 1] : s_cost[E - 1] + (i - E) * csh; },
+        (long)s_cost[E - 1] + (long)to.n_shared * csh, min(n, to.max_tiles), to.max_tiles, to.num_tiles);
   }
 }
 
