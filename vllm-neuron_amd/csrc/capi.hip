@@ -5,6 +5,7 @@
 
 #include <mutex>
 
+#include "gemm_mid.h"
 #include "moe_common.h"
 #include "moe_internal.h"
 
@@ -188,7 +189,41 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   const long NB = (long)N * B;
   const long R = routed_rows(T, K, E);
   MOE_CHECK_SUPPORTED(NB + (long)n_shared * T < (1L << 31), "too many slots");
-  const int mt = choose_mt(T, K, E);
+  // operands of the mid-size kernels
+  MidArgs mg{}, md{};
+  mg.a = w.xq;
+  mg.as = w.xs;
+  mg.w = w13;
+  mg.ws = w13_scale;
+  mg.wsh = w13_shared;
+  mg.wssh = w13_shared_scale;
+  mg.tpid = w.tpid;
+  mg.tiles = (const int4*)w.tiles;
+  mg.seg = (const int2*)w.btiles;
+  mg.num_tiles = w.bnum;
+  mg.hq = w.hq;
+  mg.hs = w.hs;
+  mg.T = T;
+  mg.H = H;
+  mg.I = I;
+  mg.E = E;
+  mg.nsh = n_shared;
+  mg.NB = NB;
+  mg.rows = R + (long)n_shared * T;
+  md = mg;
+  md.a = w.hq;
+  md.as = w.hs;
+  md.w = w2;
+  md.ws = w2_scale;
+  md.wsh = w2_shared;
+  md.wssh = w2_shared_scale;
+  md.y = w.y;
+  const bool mid_ok = mid_fits(0, mg) && mid_fits(1, md);
+  int mt = choose_mt(T, K, E);
+  // where the mid-size kernels run both heights, 64 rows keep nearly every expert in one tile
+  if (mid_ok && mt == 32 &&
+      (long)moe_max_tiles(T, K, E, N, B, n_shared, kMidTileRows) * (I / 128) >= kMidMinItems)
+    mt = kMidTileRows;
   const int max_tiles = moe_max_tiles(T, K, E, N, B, n_shared, mt);
   float* logits = logits_out ? logits_out : w.logits;
   int32_t* ids = ids_out ? ids_out : w.ids;
@@ -206,8 +241,21 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   // The mapping also writes the expert tile list, from the counts.
   const bool block = use_block(T, K, E);
   const int mbt = block ? moe_max_block_tiles(T, K, E, N, B, n_shared) : 0;
+  // Above 32 and up to kMidMaxRows rows per expert on average, 64-row block tiles: their list
+  // goes into the row-tile list's room (sized for 64-row tiles), its segments (8 bytes each)
+  // into the block tiles' (24 bytes each).
+  const int mmt = block ? mid_max_tiles(T, K, E, n_shared) : 0;
+  const bool mid = block && R <= kMidMaxRows * (long)E && mid_ok && (long)mmt * (I / 128) >= kMidMinItems &&
+                   mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) && mmt <= 3L * mbt;
   TileOut to{};
-  if (block) {
+  if (mid) {
+    to.tiles = (int4*)w.tiles;
+    to.seg = (int2*)w.btiles;
+    to.num_tiles = w.bnum;
+    to.max_tiles = mmt;
+    to.mt = kMidTileRows;
+    to.span = 1;
+  } else if (block) {
     to.tiles = (int4*)w.btiles;
     to.seg = (int2*)(w.btiles + 4 * (size_t)mbt);
     to.num_tiles = w.bnum;
@@ -244,7 +292,12 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
                                w.inv, nullptr, w.map_ws, w.map_ws_bytes, to, stream));
   // (with the norm the quantization is always done: in the logits launch or by the norm)
   if (!fz.quant_done) MOE_STEP(moe_act_quant_1x128(x_bf16, T, H, w.xq, w.xs, stream));
-  if (block) {
+  if (mid) {
+    MOE_CHECK_ARG(n_shared == 0 || (w13_shared && w13_shared_scale && w2_shared && w2_shared_scale),
+                  "shared weights missing");
+    launch_mid(0, mg, mmt, (hipStream_t)stream);
+    launch_mid(1, md, mmt, (hipStream_t)stream);
+  } else if (block) {
     MOE_STEP(moe_expert_gate_up_block(w.xq, w.xs, T, H, I, E, w13, w13_scale, nullptr, w13_shared,
                                       w13_shared_scale, nullptr, n_shared, w.tpid, (int)NB, w.btiles,
                                       w.bnum, mbt, w.hq, w.hs, stream));

@@ -29,6 +29,7 @@
 // [(l/16)*16, +16) and [64 + (l/16)*16, +16) of the K block. A and B use the
 // same mapping, so the hardware's K order inside the block does not matter.
 // Accumulator layout: lane l, register i holds D[4*(l/16) + i][l%16].
+#include "gemm_mid.h"
 #include "moe_common.h"
 #include "moe_internal.h"
 
@@ -449,6 +450,45 @@ __global__ void selftest_mfma_kernel(const uint8_t* a, const uint8_t* b, float* 
 
 template <int KIND>
 static int launch_gemm(const GemmArgs& a, int max_tiles, int mt, hipStream_t st) {
+  // Tiles of up to 64 rows run the mid-size kernels (three workgroups per CU, the same output
+  // bits): whole layer, ring kernels -> mid-size kernels, DeepSeek-V3 at 257 / 600 / 1000
+  // tokens 1850 / 2050 / 2290 -> 1769 / 1841 / 1955 us, GLM-4.5 at 100 / 500 tokens 667 / 893
+  // -> 610 / 681 us, Kimi-K2 at 600 / 1200 tokens 2857 / 3340 -> 2660 / 2841 us. 16- and 32-row
+  // tiles only where the items fill the chip twice (GLM-4.5 4 / 30 tokens 160 / 503 -> 147 /
+  // 481 us, DeepSeek-V3 16 tokens 723 -> 688 us, 64 tokens 1472 -> 1427 us): below that an item
+  // is a chain of K steps, which the ring's three stages shorten (DeepSeek-V3 2 tokens, 272
+  // items: 133 against 158 us; the small layer's 32 items at 64 tokens: 36.6 against 37.5 us).
+  // The ring at 64 rows (four fragments per wave and step) loses there too (small layer at
+  // 100 tokens 49 against 41 us).
+  const long items_mid = (long)max_tiles * ((KIND == 0) ? a.I / 128 : a.H / 256);
+  if (mt == 64 || (mt <= 32 && items_mid >= kMidMinItems)) {
+    MidArgs m{};
+    m.a = a.a;
+    m.as = a.as;
+    m.w = a.w;
+    m.ws = a.ws;
+    m.wsh = a.wsh;
+    m.wssh = a.wssh;
+    m.tpid = a.tpid;
+    m.tiles = a.tiles;
+    m.num_tiles = a.num_tiles;
+    m.hq = a.hq;
+    m.hs = a.hs;
+    m.y = a.y;
+    m.cs = a.cs;
+    m.cssh = a.cssh;
+    m.T = a.T;
+    m.H = a.H;
+    m.I = a.I;
+    m.E = a.E;
+    m.nsh = a.nsh;
+    m.NB = a.NB;
+    m.rows = a.NB + (long)a.nsh * a.T;
+    if (mid_fits(KIND, m)) {
+      launch_mid(KIND, m, max_tiles, st);
+      return MOE_OK;
+    }
+  }
   // down at 16 and 32 rows: 128 weight rows per workgroup (2 waves), so two
   // workgroups share a CU and one's start-up overlaps the other's weight stream
   constexpr int NWD = (KIND == 1) ? 2 : 4;

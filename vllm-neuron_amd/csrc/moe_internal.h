@@ -28,6 +28,16 @@ constexpr int kBlockTileRows = 256;
 // Rows per tile of the prefill-sized MXFP4 expert GEMM kernels.
 constexpr int kMxBlockTileRows = 128;
 
+// Rows per tile of the mid-size fp8 expert GEMM kernels (gemm_fp8_mid.hip). The layer runs
+// them instead of the block kernels from 32 up to kMidMaxRows routed rows per expert on
+// average: layer, block -> mid-size kernels, at 33 rows DeepSeek-V3 2127 -> 2020 us and Kimi-K2
+// 3134 -> 3051 us, at 35 GLM-4.5 805 -> 741 us; at 41 DeepSeek-V3 2165 -> 2158 us; at 50 and
+// above, where experts take two 64-row tiles, they lose (DeepSeek-V3 2241 -> 2294 us).
+constexpr int kMidTileRows = 64;
+constexpr int kMidMaxRows = 40;
+// Work items (two per CU) from which they run 16-row tiles and small layers.
+constexpr long kMidMinItems = 512;
+
 // Compute units of the current device (cached per device; 256 on MI355X), for
 // persistent grids of one workgroup per CU.
 inline int device_cu_count() {
@@ -146,6 +156,9 @@ int layer_down_combine_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, in
                           int wfmt, const uint8_t* w2, const uint8_t* w2_scale, const float* b2,
                           const int32_t* ids, const int32_t* inv, const float* weights,
                           void* out_bf16, void* stream, bool* done);
+
+// Most block tiles of kMidTileRows rows that the layer's mapping writes (compact rows).
+int mid_max_tiles(int T, int K, int E, int n_shared);
 
 // The prefill-sized MXFP4 expert GEMMs (gemm_mx_block.hip) for the layer, on block tiles
 // of kMxBlockTileRows rows (compact rows, no shared experts; at most mx_block_max_tiles
