@@ -1,8 +1,9 @@
-"""The prefill-sized MXFP4 expert GEMMs of the layer (above 32 routed rows per expert).
+"""The MXFP4 block kernels: of the layer above 32 routed rows per expert (block tiles), and of
+32- and 64-row tiles of at least 512 work items.
 
-Same scaled MFMAs in the same K order and the same epilogue arithmetic as the row-tile
-kernels, so the layer's output is held bit for bit to the op-by-op path, which runs the
-row-tile kernels (those are checked against the oracle in test_gpu_mx.py)."""
+Same scaled MFMAs in the same K order and the same epilogue arithmetic as the ring kernels,
+so results are held bit for bit to those on 16-row tiles, which always run them (and which
+test_gpu_mx.py checks against the oracle)."""
 import dataclasses
 
 import pytest
@@ -19,6 +20,20 @@ def _skew(w, counts_bias):
     return dataclasses.replace(w, router_bias=torch.tensor(counts_bias, device=w.w13.device))
 
 
+def _ring_experts(x, ids, wts, w, act, gl, ul, B=256):
+    """ops.mx_experts on 16-row tiles."""
+    T, K = ids.shape
+    E, H = w.n_experts, w.hidden
+    m = ops.blockwise_mapping(ids=ids.contiguous(), n_experts=E, top_k=K, block_size=B)
+    tpid, b2e = m["token_position_to_id"], m["block_to_expert"]
+    NB = tpid.numel()
+    xq, xs = ops.act_quant_mx(x)
+    tiles, num, mx = ops.build_tiles(tpid, b2e, B, T, K, E, 0, 16)
+    hq, hs = ops.expert_gate_up_mx(xq, xs, w, tpid, NB, tiles, num, mx, 16, NB, act, gl, ul)
+    y = ops.expert_down_mx(hq, hs, w, T, NB, tiles, num, mx, 16)
+    return ops.combine(y, m["inv_pos"], wts.contiguous(), T, H, NB, 0)
+
+
 # T * K / E > 32 in all of them. H = I = 512: one scale group, two steps; 1536 x 1024: odd
 # numbers of groups; 768: not a multiple of 512, which stays on the row-tile kernels.
 @pytest.mark.parametrize("T,E,K,H,I,act,bias,skew", [
@@ -30,7 +45,7 @@ def _skew(w, counts_bias):
     (1025, 16, 4, 1024, 1024, "swish", True, [0.0] * 16),
     (300, 8, 2, 768, 512, "swish", True, [0.0] * 8),
 ])
-def test_layer_equals_row_tile_path(cuda, T, E, K, H, I, act, bias, skew):
+def test_layer_equals_ring_kernels(cuda, T, E, K, H, I, act, bias, skew):
     say("mx block layer", T, E, K, H, I, act)
     w = _skew(make_mx_weights(E, H, I, 11, cuda, bias=bias), skew)
     g = torch.Generator().manual_seed(T)
@@ -38,6 +53,27 @@ def test_layer_equals_row_tile_path(cuda, T, E, K, H, I, act, bias, skew):
     gl, ul = ((None, 7.0), (-6.0, 8.0)) if act == "swish" else ((None, None), (None, None))
     assert T * K > 32 * E
     out, ids, wts, _ = ops.layer_forward_mx(x, w, K, act, gl, ul, return_routing=True)
-    ref = ops.mx_experts(x, ids, wts, w, act, gl, ul)
+    ref = _ring_experts(x, ids, wts, w, act, gl, ul)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     assert bool(torch.isfinite(out.float()).all()) and float(out.float().abs().max()) > 0
+
+
+# 5 to 32 rows per expert: row tiles (the layer's, and the operator path's at 32 or 64 rows).
+@pytest.mark.parametrize("T,E,K,H,I,act,B", [
+    (160, 128, 4, 512, 512, "swish", 256),
+    (700, 160, 4, 512, 1024, "silu", 256),
+    (900, 128, 4, 1024, 512, "swish", 16),   # 16-slot blocks: every tile at most 16 rows
+    (200, 40, 4, 512, 512, "swish", 256),    # too few items: the ring kernels
+])
+def test_row_tiles_equal_ring_kernels(cuda, T, E, K, H, I, act, B):
+    say("mx block row tiles", T, E, K, H, I, act, B)
+    w = make_mx_weights(E, H, I, 13, cuda)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(cuda)
+    gl, ul = ((None, 7.0), (-6.0, 8.0)) if act == "swish" else ((None, None), (None, None))
+    assert 4 * E < T * K <= 32 * E
+    out, ids, wts, _ = ops.layer_forward_mx(x, w, K, act, gl, ul, return_routing=True, block_size=B)
+    ref = _ring_experts(x, ids, wts, w, act, gl, ul, B)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    got = ops.mx_experts(x, ids, wts, w, act, gl, ul, block_size=B)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))

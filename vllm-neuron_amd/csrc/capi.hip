@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "gemm_mid.h"
+#include "gemm_mx.h"
 #include "moe_common.h"
 #include "moe_internal.h"
 
@@ -442,7 +443,43 @@ extern "C" int moe_layer_forward_mx(
   const long NB = (long)N * B;
   const long R = routed_rows(T, K, E);
   MOE_CHECK_SUPPORTED(NB < (1L << 31), "too many slots");
-  const int mt = choose_mt_mx(T, K, E);
+  // operands of the block kernels
+  MxArgs bg{}, bd{};
+  bg.a = w.xq;
+  bg.as = (const uint8_t*)w.xs;
+  bg.w = w13;
+  bg.ws = w13_scale;
+  bg.bias = b13;
+  bg.tpid = w.tpid;
+  bg.tiles = (const int4*)w.tiles;
+  bg.seg = (const int2*)w.btiles;
+  bg.num_tiles = w.bnum;
+  bg.hq = w.hq;
+  bg.hs = (uint8_t*)w.hs;
+  bg.T = T;
+  bg.H = H;
+  bg.I = I;
+  bg.E = E;
+  bg.NB = NB;
+  bg.rows = R;
+  auto lim = [](float v, float dflt) { return v != v ? dflt : v; };  // NaN: no limit
+  bg.act = act;
+  bg.gate_lo = lim(gate_lo, -__builtin_inff());
+  bg.gate_hi = lim(gate_hi, __builtin_inff());
+  bg.up_lo = lim(up_lo, -__builtin_inff());
+  bg.up_hi = lim(up_hi, __builtin_inff());
+  bd = bg;
+  bd.a = w.hq;
+  bd.as = (const uint8_t*)w.hs;
+  bd.w = w2;
+  bd.ws = w2_scale;
+  bd.bias = b2;
+  bd.y = w.y;
+  const bool block_ok = wfmt == MOE_MX_FP4 && (act == MOE_ACT_SILU || act == MOE_ACT_SWISH) &&
+                        mx_block_fits(0, bg) && mx_block_fits(1, bd);
+  int mt = choose_mt_mx(T, K, E);
+  // where the block kernels run both heights, 64 rows keep nearly every expert in one tile
+  if (block_ok && mt == 32 && (long)moe_max_tiles(T, K, E, N, B, 0, 64) * (I / 128) >= kMidMinItems) mt = 64;
   const int max_tiles = moe_max_tiles(T, K, E, N, B, 0, mt);
   float* logits = logits_out ? logits_out : w.logits;
   int32_t* ids = ids_out ? ids_out : w.ids;
@@ -463,7 +500,7 @@ extern "C" int moe_layer_forward_mx(
   // into the row-tile list's room (at most R / 128 + E of them, which is no more than the
   // R / 64 + N row tiles it is sized for, N >= E), their segments (8 bytes each) into the
   // fp8 block tiles' (24 bytes for each of NB / 256 + E, NB >= R).
-  const bool block = use_block(T, K, E) && mx_block_ok(T, H, I, E, K, wfmt, w13, w13_scale, w2, w2_scale);
+  const bool block = use_block(T, K, E) && block_ok;
   const int mbt = block ? mx_block_max_tiles(T, K, E) : 0;
   TileOut to{};
   to.tiles = (int4*)w.tiles;
@@ -504,10 +541,8 @@ extern "C" int moe_layer_forward_mx(
                                w.inv, nullptr, w.map_ws, w.map_ws_bytes, to, stream));
   if (!fz.quant_done) MOE_STEP(moe_act_quant_mx(xr, T, H, w.xq, xs, stream));
   if (block) {
-    MOE_STEP(layer_gate_up_mx_block(w.xq, xs, T, H, I, E, w13, w13_scale, b13, w.tpid, w.tiles, w.btiles,
-                                    w.bnum, mbt, act, gate_lo, gate_hi, up_lo, up_hi, w.hq, hs, stream));
-    MOE_STEP(layer_down_mx_block(w.hq, hs, T, H, I, E, w2, w2_scale, b2, w.tiles, w.btiles, w.bnum, mbt,
-                                 R, w.y, stream));
+    launch_mx_block(0, bg, mbt, (hipStream_t)stream);
+    launch_mx_block(1, bd, mbt, (hipStream_t)stream);
     MOE_STEP(moe_combine(w.y, w.inv, wts, K, T, H, (int)R, 0, out_bf16, stream));
     return MOE_OK;
   }

@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "moe_common.h"
+#include "moe_internal.h"
 
 namespace moe {
 
@@ -32,8 +33,19 @@ struct MxArgs {
   float gate_lo, gate_hi, up_lo, up_hi;
   // the layer at one token (tiles from its own mapping: one row each, token 0)
   int one;
-  long rows;  // rows of h (block kernels)
+  // block kernels: rows of h, and {first tile of the expert, tiles of the expert} of block
+  // tiles (null: row tiles)
+  long rows;
+  const int2* seg;
 };
+
+// Launch of the MXFP4 block kernels (gemm_mx_block.hip; kind 0 gate_up, 1 down) on a.tiles:
+// block tiles (a.seg set, XCD ranges in the header num_tiles) or row tiles, of at most
+// kMxBlockTileRows rows. mx_block_fits: the sizes and operands suit them (H and I multiples
+// of 512, no shared experts, 16-byte aligned operands that 32-bit byte offsets reach).
+bool mx_block_fits(int kind, const MxArgs& a);
+void launch_mx_block(int kind, const MxArgs& a, int max_tiles, hipStream_t st);
+
 
 __device__ __forceinline__ v4f mfma_mx(const v8i& a, const v8i& b, const v4f& c, int sa, int sb,
                                       std::integral_constant<int, kFmtFp8>) {

@@ -835,6 +835,19 @@ __global__ __launch_bounds__(64 * kDownCombineMaxK) void down_combine_mx_one_ker
 
 template <int KIND, int WFMT>
 static int launch_mx(const MxArgs& a, int max_tiles, int mt, hipStream_t st) {
+  // MXFP4 tiles of 32 and 64 rows, enough of them to fill the chip twice: the block kernels
+  // (two workgroups per CU, the same output bits). GPT-OSS-120B layer, ring -> block kernels:
+  // 160 tokens 380 -> 329 us, 512 424 -> 361 us, 1000 534 -> 402 us; at 16-row tiles the ring
+  // is the faster (128 tokens 316 against 325 us, 48 tokens 270 against 281 us).
+  if (WFMT == kFmtFp4 && (mt == 32 || mt == 64) &&
+      (long)max_tiles * ((KIND == 0) ? a.I / 128 : a.H / 256) >= kMidMinItems) {
+    MxArgs b = a;
+    b.rows = a.NB;
+    if (mx_block_fits(KIND, b)) {
+      launch_mx_block(KIND, b, max_tiles, st);
+      return MOE_OK;
+    }
+  }
   // The layer at one token with MXFP4 weights and K = 3072: the register kernel, one
   // workgroup per work item. Gate_up items are two MX blocks of h (196 KB of weight
   // rows), down items 64 output columns (98 KB): the time follows the bytes of the

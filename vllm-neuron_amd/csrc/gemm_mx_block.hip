@@ -45,11 +45,6 @@ constexpr int kMbThreads = 256;
 constexpr int kMbHalfA = kMbRows * 128;
 static_assert(kMbRows == kMxBlockTileRows, "tile rows");
 
-struct MxBlkArgs {
-  MxArgs m;
-  const int2* seg;  // {first tile of the expert, tiles of the expert}
-};
-
 struct MbLds {
   uint8_t* b;      // weight tile of the step: 256 rows x 128 bytes
   uint8_t* a;      // token rows, first and second 128 K values of the step (16 KB each)
@@ -379,27 +374,33 @@ __device__ __forceinline__ void mx_block_item(const MxArgs& p, const MbLds& s, c
   }
 }
 
+// Block tiles (p.seg set) or row tiles.
 template <int KIND>
-__global__ __launch_bounds__(kMbThreads, 2) void expert_gemm_mx_block_kernel(MxBlkArgs a) {
+__global__ __launch_bounds__(kMbThreads, 2) void expert_gemm_mx_block_kernel(MxArgs p) {
   __shared__ __attribute__((aligned(1024))) uint8_t sB[kMbCols * 128];
   __shared__ __attribute__((aligned(1024))) uint8_t sA[2 * kMbHalfA];
   __shared__ __attribute__((aligned(1024))) uint8_t sBS[2 * kMbCols * 16];
   __shared__ __attribute__((aligned(1024))) uint8_t sAS[2 * kMbRows * 16];
   __shared__ int sTok[kMbRows];
   const MbLds s{sB, sA, sBS, sAS, sTok};
-  const MxArgs& p = a.m;
-  // XCD-aware item index, as in the fp8 block kernels: XCD x takes the items of tiles
-  // [cut[x], cut[x + 1]) of the list's header, expert by expert and column tile by
-  // column tile, so the row tiles of an expert share each weight tile in one L2.
   const int NT = (KIND == 0) ? p.I / 128 : p.H / kMbCols;
-  const int x = blockIdx.x & 7;
-  const int L = p.num_tiles[1 + x] * NT + (int)(blockIdx.x >> 3);
-  if (L >= p.num_tiles[2 + x] * NT) return;
-  const int2 sg = a.seg[L / NT];
-  const int r0 = L - NT * sg.x;
-  const int nt = r0 / sg.y;
-  const int tile = sg.x + (r0 - nt * sg.y);
-  if (tile >= p.num_tiles[0]) return;  // truncated tile list
+  int tile, nt;
+  if (p.seg != nullptr) {
+    // XCD-aware item index, as in the fp8 block kernels: XCD x takes the items of tiles
+    // [cut[x], cut[x + 1]) of the list's header, expert by expert and column tile by
+    // column tile, so the row tiles of an expert share each weight tile in one L2.
+    const int x = blockIdx.x & 7;
+    const int L = p.num_tiles[1 + x] * NT + (int)(blockIdx.x >> 3);
+    if (L >= p.num_tiles[2 + x] * NT) return;
+    const int2 sg = p.seg[L / NT];
+    const int r0 = L - NT * sg.x;
+    nt = r0 / sg.y;
+    tile = sg.x + (r0 - nt * sg.y);
+  } else {
+    tile = blockIdx.x / NT;
+    nt = blockIdx.x - tile * NT;
+  }
+  if (tile >= p.num_tiles[0]) return;  // past the list, or a truncated one
   // (wave-uniform, so the operand bases stay in scalar registers)
   const int4 tv = p.tiles[tile];
   const int4 td = make_int4(__builtin_amdgcn_readfirstlane(tv.x), __builtin_amdgcn_readfirstlane(tv.y),
@@ -418,88 +419,28 @@ __global__ __launch_bounds__(kMbThreads, 2) void expert_gemm_mx_block_kernel(MxB
   }
 }
 
-template <int KIND>
-static void launch_mx_block(const MxBlkArgs& a, int max_tiles, hipStream_t st) {
-  const int NT = (KIND == 0) ? a.m.I / 128 : a.m.H / kMbCols;
-  const long items = 8L * block_tiles_cap(max_tiles) * NT;  // each XCD's share of the tiles
-  hipLaunchKernelGGL(expert_gemm_mx_block_kernel<KIND>, dim3((unsigned)items), dim3(kMbThreads), 0, st, a);
+bool mx_block_fits(int kind, const MxArgs& a) {
+  auto al = [](const void* q, uintptr_t n) { return ((uintptr_t)q & (n - 1)) == 0; };
+  const unsigned long lim = 1UL << 32;
+  return a.nsh == 0 && a.H % 512 == 0 && a.I % 512 == 0 && al(a.a, 16) && al(a.as, 16) && al(a.w, 16) &&
+         al(a.ws, 16) && al(a.hq, 2) && al(a.y, 8) &&
+         (unsigned long)(kind == 0 ? a.T : a.rows) * (unsigned long)(kind == 0 ? a.H : a.I) < lim &&
+         (unsigned long)a.I * a.H < lim && a.rows < (1L << 31);
+}
+
+void launch_mx_block(int kind, const MxArgs& a, int max_tiles, hipStream_t st) {
+  const long NT = (kind == 0) ? a.I / 128 : a.H / kMbCols;
+  // block tiles: each XCD's share of them
+  const long items = (a.seg != nullptr ? 8L * block_tiles_cap(max_tiles) : (long)max_tiles) * NT;
+  if (kind == 0)
+    hipLaunchKernelGGL(expert_gemm_mx_block_kernel<0>, dim3((unsigned)items), dim3(kMbThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(expert_gemm_mx_block_kernel<1>, dim3((unsigned)items), dim3(kMbThreads), 0, st, a);
 }
 
 }  // namespace moe
 
-using namespace moe;
-
 int moe::mx_block_max_tiles(int T, int K, int E) {
   const long rows = (long)T * std::min(K, E);
   return (int)(rows / kMxBlockTileRows + std::min<long>(E, rows));
-}
-
-bool moe::mx_block_ok(int T, int H, int I, int E, int K, int wfmt, const void* w13,
-                      const void* w13_scale, const void* w2, const void* w2_scale) {
-  const unsigned long rows = (unsigned long)T * std::min(K, E);
-  auto a16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-  return wfmt == MOE_MX_FP4 && H % 512 == 0 && I % 512 == 0 && a16(w13) && a16(w13_scale) && a16(w2) &&
-         a16(w2_scale) && (unsigned long)T * H < (1UL << 32) && rows * I < (1UL << 32) &&
-         (unsigned long)I * H < (1UL << 32);
-}
-
-int moe::layer_gate_up_mx_block(const uint8_t* xq, const uint8_t* xs, int T, int H, int I, int E,
-                                const uint8_t* w13, const uint8_t* w13_scale, const float* b13,
-                                const int32_t* token_position_to_id, const int32_t* tiles,
-                                const int32_t* seg, const int32_t* num_tiles, int max_tiles, int act,
-                                float gate_lo, float gate_hi, float up_lo, float up_hi, uint8_t* hq,
-                                uint8_t* hs, void* stream) {
-  MOE_API_BEGIN("moe_expert_gate_up_mx");
-  MOE_CHECK_ARG(xq && xs && w13 && w13_scale && token_position_to_id && tiles && seg && num_tiles && hq && hs,
-                "null pointer argument");
-  MOE_CHECK_ARG(act == MOE_ACT_SILU || act == MOE_ACT_SWISH, "act must be MOE_ACT_SILU or MOE_ACT_SWISH");
-  auto lim = [](float v, float dflt) { return v != v ? dflt : v; };
-  MxBlkArgs a{};
-  a.m.a = xq;
-  a.m.as = xs;
-  a.m.w = w13;
-  a.m.ws = w13_scale;
-  a.m.bias = b13;
-  a.m.tpid = token_position_to_id;
-  a.m.tiles = (const int4*)tiles;
-  a.m.num_tiles = num_tiles;
-  a.m.hq = hq;
-  a.m.hs = hs;
-  a.m.T = T;
-  a.m.H = H;
-  a.m.I = I;
-  a.m.E = E;
-  a.m.act = act;
-  a.m.gate_lo = lim(gate_lo, -__builtin_inff());
-  a.m.gate_hi = lim(gate_hi, __builtin_inff());
-  a.m.up_lo = lim(up_lo, -__builtin_inff());
-  a.m.up_hi = lim(up_hi, __builtin_inff());
-  a.seg = (const int2*)seg;
-  launch_mx_block<0>(a, max_tiles, (hipStream_t)stream);
-  MOE_API_END();
-}
-
-int moe::layer_down_mx_block(const uint8_t* hq, const uint8_t* hs, int T, int H, int I, int E,
-                             const uint8_t* w2, const uint8_t* w2_scale, const float* b2,
-                             const int32_t* tiles, const int32_t* seg, const int32_t* num_tiles,
-                             int max_tiles, long rows, void* y_bf16, void* stream) {
-  MOE_API_BEGIN("moe_expert_down_mx");
-  MOE_CHECK_ARG(hq && hs && w2 && w2_scale && tiles && seg && num_tiles && y_bf16, "null pointer argument");
-  MxBlkArgs a{};
-  a.m.a = hq;
-  a.m.as = hs;
-  a.m.w = w2;
-  a.m.ws = w2_scale;
-  a.m.bias = b2;
-  a.m.tiles = (const int4*)tiles;
-  a.m.num_tiles = num_tiles;
-  a.m.y = (uint16_t*)y_bf16;
-  a.m.rows = rows;
-  a.m.T = T;
-  a.m.H = H;
-  a.m.I = I;
-  a.m.E = E;
-  a.seg = (const int2*)seg;
-  launch_mx_block<1>(a, max_tiles, (hipStream_t)stream);
-  MOE_API_END();
 }

@@ -160,24 +160,8 @@ int layer_down_combine_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, in
 // Most block tiles of kMidTileRows rows that the layer's mapping writes (compact rows).
 int mid_max_tiles(int T, int K, int E, int n_shared);
 
-// The prefill-sized MXFP4 expert GEMMs (gemm_mx_block.hip) for the layer, on block tiles
-// of kMxBlockTileRows rows (compact rows, no shared experts; at most mx_block_max_tiles
-// of them) that its own mapping wrote. mx_block_ok: the operands suit them (MXFP4
-// weights, H and I multiples of 512, 16-byte aligned weights and scales, operands that
-// 32-bit byte offsets reach); otherwise the layer runs the row-tile kernels.
-bool mx_block_ok(int T, int H, int I, int E, int K, int wfmt, const void* w13, const void* w13_scale,
-                 const void* w2, const void* w2_scale);
+// Most block tiles of kMxBlockTileRows rows that the layer's mapping writes (compact rows).
 int mx_block_max_tiles(int T, int K, int E);
-int layer_gate_up_mx_block(const uint8_t* xq, const uint8_t* xs, int T, int H, int I, int E,
-                           const uint8_t* w13, const uint8_t* w13_scale, const float* b13,
-                           const int32_t* token_position_to_id, const int32_t* tiles,
-                           const int32_t* seg, const int32_t* num_tiles, int max_tiles, int act,
-                           float gate_lo, float gate_hi, float up_lo, float up_hi, uint8_t* hq,
-                           uint8_t* hs, void* stream);
-int layer_down_mx_block(const uint8_t* hq, const uint8_t* hs, int T, int H, int I, int E,
-                        const uint8_t* w2, const uint8_t* w2_scale, const float* b2,
-                        const int32_t* tiles, const int32_t* seg, const int32_t* num_tiles,
-                        int max_tiles, long rows, void* y_bf16, void* stream);
 
 // moe_blockwise_mapping plus an optional tile list (same checks and errors).
 int blockwise_mapping(const int32_t* ids, const float* affinities, const uint8_t* padding_mask,
