@@ -77,3 +77,22 @@ def test_row_tiles_equal_ring_kernels(cuda, T, E, K, H, I, act, B):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     got = ops.mx_experts(x, ids, wts, w, act, gl, ul, block_size=B)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+# Above four tokens the norm's own pass writes the MXFP8 codes: the same bits as the layer
+# without its norm on the normalized rows.
+@pytest.mark.parametrize("T,residual,actual", [(5, False, 480), (77, True, 512), (600, True, 500)])
+def test_norm_pass_quantizes(cuda, T, residual, actual):
+    say("mx norm pass", T, residual, actual)
+    w = make_mx_weights(16, 512, 512, 17, cuda)
+    g = torch.Generator().manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    x, res = (rnd(T, 512).to(torch.bfloat16).to(cuda) for _ in range(2))
+    gamma = (1 + 0.1 * rnd(512)).to(cuda)
+    res = res if residual else None
+    got = ops.layer_forward_mx(x, w, 4, gamma=gamma, eps=1e-5, hidden_actual=actual, residual=res)
+    out, rsum = got if residual else (got, None)
+    xn, _, _, v = ops.rms_norm_quant(x, gamma, 1e-5, actual, res)
+    ref = ops.layer_forward_mx(xn, w, 4)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    assert rsum is None or torch.equal(rsum.view(torch.int16), v.view(torch.int16))

@@ -520,7 +520,7 @@ extern "C" int moe_layer_forward_mx(
   to.compact = 1;
   to.row_shared = R;
   // Residual add + RMSNorm: up to a few tokens inside the logits launch, else in a
-  // pass of its own before it (whose 1x128 codes land in xq and are replaced below).
+  // pass of its own before it, which quantizes the normalized rows too.
   // Decode sizes: the MXFP8 quantization rides in the logits launch and the
   // mapping ends the top-k launch (router_logits_topk says which it did).
   RouterFuse fz = map_fuse(w, B, N, to);

@@ -98,8 +98,8 @@ constexpr int kNormRideMaxH = 16384;
 // ids it selects (when tpid is set; ids only, no padding mask, inv_pos = inv,
 // workspace map_ws, tile list `to`). With norm.gamma set, x is normalized first:
 // inside the logits launch where it can ride (then the quantization rides too),
-// otherwise by moe_rms_norm_quant into xn (its 1x128 codes land in xq / xs), which
-// the router then reads. On return quant_done / map_done say which it did; the
+// otherwise by rms_norm_quant into xn (its codes land in xq / xs), which the router then
+// reads. On return quant_done / map_done say which it did; the
 // caller runs the rest itself (from xn when the norm was requested).
 struct RouterFuse {
   uint8_t* xq;
@@ -114,6 +114,11 @@ struct RouterFuse {
   TileOut to;
   bool quant_done, map_done;
 };
+
+// moe_rms_norm_quant, or with mx the same pass with MXFP8 codes in q and E8M0 scale bytes in s.
+int rms_norm_quant(const void* x_bf16, const void* residual_bf16, const float* gamma, int T, int H,
+                   int hidden_actual, float eps, void* xn_bf16, void* residual_out_bf16, uint8_t* q,
+                   void* s, bool mx, void* stream);
 
 // moe_router_logits followed by moe_router_topk (no affinities output), with the
 // split-K reduce folded into the top-k kernel; for callers that already checked

@@ -11,6 +11,8 @@
 // router.py:236 casts hidden_states to the computation dtype (fp32) before the
 // optional RMSNorm, so with gamma (or fp32 inputs) F.linear runs on fp32
 // operands (router.py:418-424). It uses v_mfma_f32_16x16x4f32.
+#include <type_traits>
+
 #include "moe_common.h"
 #include "moe_internal.h"
 
@@ -56,12 +58,15 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const void* __restrict__ 
 // The sum of squares runs in a fixed order: each thread over its chunks and their 8
 // values in order, a wave butterfly, then the four wave sums in order.
 // RES: the row is first v = bf16(x + residual) (written to res_out: the next residual
-// stream). QUANT (H % 128 == 0): the bf16 normalized row is also quantized 1x128 to
-// e4m3fn, one group per 16-lane segment, with act_quant's arithmetic. rms_norm and the
-// fused prologue both run this kernel, so the prologue's normalized row is bit-identical
-// to moe_rms_norm's and its codes to moe_act_quant_1x128 of that row.
+// stream). QUANT (H % 128 == 0): the bf16 normalized row is also quantized, 1 to e4m3fn with
+// 1x128 scales, one group per 16-lane segment, with act_quant's arithmetic, 2 to MXFP8, one
+// block per 4-lane group, with mx_act_quant's. rms_norm and the fused prologue both run this
+// kernel, so the prologue's normalized row is bit-identical to moe_rms_norm's and its codes
+// to moe_act_quant_1x128 (moe_act_quant_mx) of that row. HBM-bound: GPT-OSS-120B, 8192 rows
+// with the residual, 226 MB in 40 us; the MXFP8 codes as a pass of their own took 12.7 us
+// more (5.6 us at 2048 rows). The whole layer: 1111 to 1092 us at 8192 rows, 481 to 480 at 2048.
 constexpr int kNormMaxChunks = 8;  // H <= 256 * 8 * 8 = 16384
-template <bool XF32, bool OF32, bool RES, bool QUANT, int NJ>
+template <bool XF32, bool OF32, bool RES, int QUANT, int NJ>
 __global__ __launch_bounds__(256) void rms_norm_vec_kernel(
     const void* __restrict__ x, const uint16_t* __restrict__ res, const float* __restrict__ gamma,
     int H, int ha, float eps, void* __restrict__ out, uint16_t* __restrict__ res_out,
@@ -124,7 +129,10 @@ __global__ __launch_bounds__(256) void rms_norm_vec_kernel(
           yb[2 * i] = __uint_as_float(w[i] << 16);
           yb[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
         }
-        quant8_1x128(yb, q + base + 8 * c, qs + (size_t)blockIdx.x * G + (c >> 4), (tid & 15) == 0);
+        if constexpr (QUANT == 1)
+          quant8_1x128(yb, q + base + 8 * c, qs + (size_t)blockIdx.x * G + (c >> 4), (tid & 15) == 0);
+        else  // whole 4-lane groups hold a 32-value block
+          mx_quant_chunk(yb, true, (long)blockIdx.x * nch + c, q, (uint8_t*)qs);
       }
     }
   }
@@ -235,7 +243,7 @@ __global__ void router_logits_f32_reduce(const float* __restrict__ part,
 }
 
 // Launch rms_norm_vec_kernel with the smallest chunk count per thread that covers H.
-template <bool XF32, bool OF32, bool RES, bool QUANT>
+template <bool XF32, bool OF32, bool RES, int QUANT>
 static void launch_rms_norm_vec(int T, int H, hipStream_t st, const void* x, const uint16_t* res,
                                 const float* gamma, int ha, float eps, void* out,
                                 uint16_t* res_out, uint8_t* q, float* qs) {
@@ -275,24 +283,24 @@ extern "C" int moe_rms_norm(const void* x, int x_is_f32, const float* gamma, int
     hipLaunchKernelGGL(rms_norm_kernel, dim3(T), dim3(256), 0, st, x, x_is_f32 ? 1 : 0, gamma, H,
                        hidden_actual, eps, out, out_is_f32 ? 1 : 0);
   } else if (x_is_f32 && out_is_f32) {
-    launch_rms_norm_vec<true, true, false, false>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
+    launch_rms_norm_vec<true, true, false, 0>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
                                                   nullptr, nullptr);
   } else if (x_is_f32) {
-    launch_rms_norm_vec<true, false, false, false>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
+    launch_rms_norm_vec<true, false, false, 0>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
                                                   nullptr, nullptr);
   } else if (out_is_f32) {
-    launch_rms_norm_vec<false, true, false, false>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
+    launch_rms_norm_vec<false, true, false, 0>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
                                                   nullptr, nullptr);
   } else {
-    launch_rms_norm_vec<false, false, false, false>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
+    launch_rms_norm_vec<false, false, false, 0>(T, H, st, x, nullptr, gamma, hidden_actual, eps, out, nullptr,
                                                   nullptr, nullptr);
   }
   MOE_API_END();
 }
 
-extern "C" int moe_rms_norm_quant(const void* x_bf16, const void* residual_bf16, const float* gamma,
-                                  int T, int H, int hidden_actual, float eps, void* xn_bf16,
-                                  void* residual_out_bf16, uint8_t* q, float* s, void* stream) {
+int moe::rms_norm_quant(const void* x_bf16, const void* residual_bf16, const float* gamma, int T, int H,
+                        int hidden_actual, float eps, void* xn_bf16, void* residual_out_bf16,
+                        uint8_t* q, void* s, bool mx, void* stream) {
   MOE_API_BEGIN("moe_rms_norm_quant");
   MOE_CHECK_ARG(x_bf16 && gamma && xn_bf16 && q && s, "null pointer argument");
   MOE_CHECK_ARG((residual_bf16 == nullptr) == (residual_out_bf16 == nullptr),
@@ -308,14 +316,26 @@ extern "C" int moe_rms_norm_quant(const void* x_bf16, const void* residual_bf16,
                     ((uintptr_t)gamma & 15) == 0 && ((uintptr_t)q & 7) == 0,
                 "x, residual, xn, residual_out and gamma must be 16-byte aligned, q 8-byte aligned");
   if (T == 0) return MOE_OK;
+  auto launch = [&](auto res_c, auto quant_c) {
+    constexpr bool RES = decltype(res_c)::value;
+    launch_rms_norm_vec<false, false, RES, decltype(quant_c)::value>(
+        T, H, (hipStream_t)stream, x_bf16, (const uint16_t*)residual_bf16, gamma, hidden_actual, eps,
+        xn_bf16, (uint16_t*)residual_out_bf16, q, (float*)s);
+  };
+  const std::integral_constant<int, 1> q1x128{};
+  const std::integral_constant<int, 2> qmx{};
   if (residual_bf16 != nullptr)
-    launch_rms_norm_vec<false, false, true, true>(T, H, (hipStream_t)stream, x_bf16,
-                                                  (const uint16_t*)residual_bf16, gamma, hidden_actual,
-                                                  eps, xn_bf16, (uint16_t*)residual_out_bf16, q, s);
+    mx ? launch(std::true_type{}, qmx) : launch(std::true_type{}, q1x128);
   else
-    launch_rms_norm_vec<false, false, false, true>(T, H, (hipStream_t)stream, x_bf16, nullptr, gamma,
-                                                   hidden_actual, eps, xn_bf16, nullptr, q, s);
+    mx ? launch(std::false_type{}, qmx) : launch(std::false_type{}, q1x128);
   MOE_API_END();
+}
+
+extern "C" int moe_rms_norm_quant(const void* x_bf16, const void* residual_bf16, const float* gamma,
+                                  int T, int H, int hidden_actual, float eps, void* xn_bf16,
+                                  void* residual_out_bf16, uint8_t* q, float* s, void* stream) {
+  return moe::rms_norm_quant(x_bf16, residual_bf16, gamma, T, H, hidden_actual, eps, xn_bf16,
+                             residual_out_bf16, q, s, false, stream);
 }
 
 extern "C" int moe_router_logits_f32(const float* x, const void* router_w, int w_is_f32,

@@ -1067,11 +1067,11 @@ int moe::router_logits_topk(const void* x_bf16, const void* w_bf16, const float*
            a16(x_bf16) && a16(nr.res) && a16(nr.res_out) && a16(nr.gamma) && fuse->xq != nullptr &&
            fuse->xs != nullptr && ((uintptr_t)fuse->xq & 7) == 0;
     if (!ride) {
-      const int rc = moe_rms_norm_quant(x_bf16, nr.res, nr.gamma, T, H, nr.ha, nr.eps, fuse->xn,
-                                        nr.res_out, fuse->xq, (float*)fuse->xs, stream);
+      const int rc = rms_norm_quant(x_bf16, nr.res, nr.gamma, T, H, nr.ha, nr.eps, fuse->xn, nr.res_out,
+                                    fuse->xq, fuse->xs, fuse->quant_mx != 0, stream);
       if (rc != MOE_OK) return rc;
       x_bf16 = fuse->xn;
-      quant_by_norm = !fuse->quant_mx;  // its 1x128 codes are the layer's
+      quant_by_norm = true;
     }
   }
   if (separate) {
