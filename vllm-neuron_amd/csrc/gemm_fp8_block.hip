@@ -565,8 +565,7 @@ __device__ __forceinline__ void block_item(const BlkArgs& p, const BlkLds& s, co
           acc[m][n][i] = h;
           mx = fmaxf(mx, fabsf(h));
         }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        mx = group16_max_f32(mx);
         if (l16 == 0) sRed[wn][row] = mx;
       }
     __syncthreads();
