@@ -70,9 +70,11 @@ def test_sixteen_row_tiles_equal_ring_kernel(cuda):
         assert torch.equal(a.view(as_int)[live], b.view(as_int)[live])
 
 
-# 33 to 40 rows per expert: the layer against the op-by-op path's block kernels. A zero weight
-# scale repeats the previous block's ratio in both.
-@pytest.mark.parametrize("T,S,zero", [(513, 1, False), (577, 0, True), (640, 1, True)])
+# 33 to 76 rows per expert: the layer against the op-by-op path's block kernels. A zero weight
+# scale repeats the previous block's ratio in both. Above 40 rows (128-row tiles) a router
+# bias spreads the experts over every count of 16-row fragments and several tiles.
+@pytest.mark.parametrize("T,S,zero", [(513, 1, False), (577, 0, True), (640, 1, True), (641, 1, False),
+                                      (1000, 0, True), (1216, 2, False)])
 def test_layer_block_tiles_equal_block_kernels(cuda, T, S, zero):
     E, K, H, I = 128, 8, 1024, 512
     cfg = MoEConfig(H, I, E, K, n_shared=S, scoring="sigmoid", grouped=True, renorm=True)
@@ -83,12 +85,20 @@ def test_layer_block_tiles_equal_block_kernels(cuda, T, S, zero):
         w.w13_scale[3, :, 2] = 0
         w.w2_scale[:, 1, 3] = 0
     x = synthetic.hidden_states(T, H, 5).to(cuda)
+    tall = T * K > 40 * E
+    if tall:
+        g = torch.Generator(device=cuda).manual_seed(6)
+        bias = torch.randn(E, device=cuda, generator=g) * (x.float() @ w.router_w.float().t()).std()
+        w = dataclasses.replace(w, router_bias=bias)
     out, ids, wts, _ = ops.layer_forward(x, w, cfg, return_routing=True)
+    if tall:
+        c = torch.bincount(ids.flatten(), minlength=E).tolist()
+        assert set(range(1, 9)) <= {-(-n // 16) for n in c} and max(c) > 128
     m = ops.blockwise_mapping(ids=ids, n_experts=E, block_size=256)
     tpid, b2e = m["token_position_to_id"], m["block_to_expert"]
     NB = tpid.numel()
     xq, xs = ops.act_quant(x)
-    assert ops.use_block_kernels(T, K, E) and T * K <= 40 * E
+    assert ops.use_block_kernels(T, K, E) and T * K <= 76 * E
     tiles, num, mx = ops.build_block_tiles(tpid, b2e, 256, T, K, E, S)
     hq, hs = ops.expert_gate_up_block(xq, xs, w, tpid, NB, tiles, num, mx)
     y = ops.expert_down_block(hq, hs, w, T, NB, tiles, num, mx)

@@ -242,11 +242,12 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   // The mapping also writes the expert tile list, from the counts.
   const bool block = use_block(T, K, E);
   const int mbt = block ? moe_max_block_tiles(T, K, E, N, B, n_shared) : 0;
-  // Above 32 and up to kMidMaxRows rows per expert on average, 64-row block tiles: their list
-  // goes into the row-tile list's room (sized for 64-row tiles), its segments (8 bytes each)
-  // into the block tiles' (24 bytes each).
-  const int mmt = block ? mid_max_tiles(T, K, E, n_shared) : 0;
-  const bool mid = block && R <= kMidMaxRows * (long)E && mid_ok && (long)mmt * (I / 128) >= kMidMinItems &&
+  // Above 32 and up to kMidTallMaxRows rows per expert on average, 64- or 128-row block
+  // tiles: their list goes into the row-tile list's room (sized for 64-row tiles), its segments
+  // (8 bytes each) into the block tiles' (24 bytes each).
+  const int mid_rows = R <= kMidMaxRows * (long)E ? kMidTileRows : kMidTallRows;
+  const int mmt = block ? mid_max_tiles(T, K, E, n_shared, mid_rows) : 0;
+  const bool mid = block && R <= kMidTallMaxRows * (long)E && mid_ok && (long)mmt * (I / 128) >= kMidMinItems &&
                    mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) && mmt <= 3L * mbt;
   TileOut to{};
   if (mid) {
@@ -254,7 +255,7 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
     to.seg = (int2*)w.btiles;
     to.num_tiles = w.bnum;
     to.max_tiles = mmt;
-    to.mt = kMidTileRows;
+    to.mt = mid_rows;
     to.span = 1;
   } else if (block) {
     to.tiles = (int4*)w.btiles;
@@ -296,8 +297,8 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   if (mid) {
     MOE_CHECK_ARG(n_shared == 0 || (w13_shared && w13_shared_scale && w2_shared && w2_shared_scale),
                   "shared weights missing");
-    launch_mid(0, mg, mmt, (hipStream_t)stream);
-    launch_mid(1, md, mmt, (hipStream_t)stream);
+    launch_mid(0, mg, mmt, mid_rows, (hipStream_t)stream);
+    launch_mid(1, md, mmt, mid_rows, (hipStream_t)stream);
   } else if (block) {
     MOE_STEP(moe_expert_gate_up_block(w.xq, w.xs, T, H, I, E, w13, w13_scale, nullptr, w13_shared,
                                       w13_shared_scale, nullptr, n_shared, w.tpid, (int)NB, w.btiles,

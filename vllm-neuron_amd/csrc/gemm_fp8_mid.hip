@@ -1,5 +1,5 @@
-// FP8-blockwise expert GEMMs on tiles of up to 64 rows, between one-token decode and prefill:
-// the weight stream sets the time.
+// FP8-blockwise expert GEMMs on tiles of up to 64 or 128 rows, between one-token decode and
+// prefill: the weight stream sets the time.
 //
 // One 16x16x128 MFMA per 128-K scale block, in the arithmetic of the kernels it stands in for,
 // so h and y are the same bits: on row tiles acc += part * (s_a[row, k] * s_w[k])
@@ -21,6 +21,14 @@
 //  * activation scales of four K blocks per row come with one 16-byte load every fourth
 //    step, weight block scales once per tile.
 //
+//  * tiles of up to 128 rows (block tiles only) keep the same step with 72 KB of LDS and 256
+//    registers, two workgroups per CU, and read the token fragments two ahead. An expert
+//    of 65 to 128 rows then reads its weights once. Layer, block -> 128-row kernels: Kimi-K2
+//    2048 tokens (43 rows per expert) 3214 -> 3129 us, GLM-4.5 1500 tokens (75) 920 -> 863 us.
+//    Tried on them: weight fragments straight to registers, without LDS (16 rows x 64 bytes a
+//    load: 3883 and 1211 us), the weight loads spread over the step (3210, 899), wave priority
+//    for the MFMAs (3134, 865).
+//
 // Measured where the rules of its use stand (gemm_fp8.hip launch_gemm, kMidMaxRows): DeepSeek-V3
 // at 600 tokens 11.3 GB of weights in a layer of 1841 us, 6.1 TB/s (ring kernels 2050 us).
 //
@@ -36,15 +44,14 @@
 
 namespace moe {
 
-constexpr int kMidRows = kMidTileRows, kMidCols = 256;
+constexpr int kMidCols = 256;
 constexpr int kMidThreads = 256;
 constexpr int kMidMaxKB = 128;  // K <= 16384
-constexpr int kMidA = kMidRows * 128;
 
 struct MidLds {
   uint8_t* b;         // weight tile: 256 rows x 128 bytes
-  uint8_t* a;         // token rows: two buffers of 64 x 128 bytes
-  uint8_t* sa;        // activation scales: two buffers of 64 rows x 4 K blocks; at the end the
+  uint8_t* a;         // token rows: two buffers of TR x 128 bytes (TR: 64 or 128 tile rows)
+  uint8_t* sa;        // activation scales: two buffers of TR rows x 4 K blocks; at the end the
                       // last block scale per (half, row)
   float (*sw)[kMidMaxKB];
   int* tok;           // token (gate_up) or h row (down) of each tile row; -1: none
@@ -70,12 +77,12 @@ struct MidFragA {
   v4i lo, hi;
   float r0, r1;
 };
-template <bool RATIO>
+template <bool RATIO, int N = 0>  // all but the newest N LDS reads
 __device__ __forceinline__ void mid_wait(MidFragA& f) {
   if constexpr (RATIO)
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.lo), "+v"(f.hi), "+v"(f.r0), "+v"(f.r1) : : "memory");
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(f.lo), "+v"(f.hi), "+v"(f.r0), "+v"(f.r1) : "n"(N) : "memory");
   else
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.lo), "+v"(f.hi), "+v"(f.r0) : : "memory");
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(f.lo), "+v"(f.hi), "+v"(f.r0) : "n"(N) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void mid_wait_b(v4i (&b)[8], float& s0, float& s1) {
@@ -87,20 +94,20 @@ __device__ __forceinline__ void mid_wait_b(v4i (&b)[8], float& s0, float& s1) {
 }
 // Token fragment m from token buffer BUF: with ratios, those of the two halves (r_addr: the
 // ratios); otherwise the tokens' scales of K block Q of the group (r_addr: the group's).
-template <int KIND, int BUF, int Q, bool RATIO>
+template <int KIND, int TR, int BUF, int Q, bool RATIO>
 __device__ __forceinline__ void mid_read_a(uint32_t lo, uint32_t hi, uint32_t r_addr, int m, MidFragA& f) {
-#define MID_A(M)                                                                              \
-  case M:                                                                                     \
-    mid_read16<kMidA * BUF + 2048 * M>(lo, f.lo);                                             \
-    mid_read16<kMidA * BUF + 2048 * M>(hi, f.hi);                                             \
-    if constexpr (RATIO) {                                                                    \
-      mid_read4<8 * kMidRows * BUF + 64 * M>(r_addr, f.r0);                                   \
-      mid_read4<8 * kMidRows * BUF + 64 * M + (KIND == 0 ? 4 * kMidRows : 0)>(r_addr, f.r1);  \
-    } else {                                                                                  \
-      mid_read4<256 * M + 4 * Q>(r_addr, f.r0);                                               \
-    }                                                                                         \
+#define MID_A(M)                                                                \
+  case M:                                                                       \
+    mid_read16<128 * TR * BUF + 2048 * M>(lo, f.lo);                            \
+    mid_read16<128 * TR * BUF + 2048 * M>(hi, f.hi);                            \
+    if constexpr (RATIO) {                                                      \
+      mid_read4<8 * TR * BUF + 64 * M>(r_addr, f.r0);                           \
+      mid_read4<8 * TR * BUF + 64 * M + (KIND == 0 ? 4 * TR : 0)>(r_addr, f.r1); \
+    } else {                                                                    \
+      mid_read4<256 * M + 4 * Q>(r_addr, f.r0);                                 \
+    }                                                                           \
     break;
-  switch (m) { MID_A(0) MID_A(1) MID_A(2) MID_A(3) }
+  switch (m) { MID_A(0) MID_A(1) MID_A(2) MID_A(3) MID_A(4) MID_A(5) MID_A(6) MID_A(7) }
 #undef MID_A
 }
 
@@ -121,10 +128,14 @@ __device__ __forceinline__ v4f mid_mfma(const v8i& w, const v8i& t, const v4f& c
 // One work item: rows [slot0, slot0 + nrows) of expert e (hq / y rows from rbase), at most
 // 16 MF of them, against column tile nt; alone: e has no
 // other row tile.
-template <int KIND, int MF, bool RATIO>
+template <int KIND, int TR, int MF, bool RATIO>
 __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, const int e, const long slot0,
                                          const long rbase, const int nrows, const int nt, const bool alone) {
-  constexpr int NA = (MF + 1) / 2;  // token-row loads per wave and step
+  constexpr int NA = (MF + 1) / 2;       // token-row loads per wave and step
+  // Token fragments in registers, read D - 1 ahead (from seven row groups on the accumulators
+  // leave room for two).
+  constexpr int D = TR > 64 && MF <= 6 ? 3 : 2;
+  constexpr int kA = TR * 128, kS = TR * 16;  // bytes of a token and of a scale buffer
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
@@ -189,7 +200,8 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     areg[i] = min(wave + 4 * i, 2 * MF - 1);  // 8-row region; past the last, the last once more
     aid[i] = id_of(8 * areg[i] + (lane >> 3));
   }
-  const int sid = id_of(lane);
+  const int srow = TR > 64 ? 64 * (wave & 1) + lane : lane;  // waves below TR / 64 load the scales
+  const int sid = id_of(srow);
   __builtin_amdgcn_sched_barrier(0);
   load_b(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -199,17 +211,17 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     const int row = 8 * areg[i] + (lane >> 3), src = src_of(row, aid[i]);
     aoff[i] = (uint32_t)(src < 0 ? 0 : src) * (uint32_t)Kdim + (uint32_t)(swz(row, lane & 7) * 16);
   }
-  const int ssrc = src_of(lane, sid);
+  const int ssrc = src_of(srow, sid);
   const uint32_t soff = (uint32_t)(ssrc < 0 ? 0 : ssrc) * (uint32_t)(KB * 4);
   auto load_a = [&](int i, int kb, int buf) {
-    buf_lds16(ra, aoff[i], kb * 128, s.a + buf * kMidA + areg[i] * 1024);
+    buf_lds16(ra, aoff[i], kb * 128, s.a + buf * kA + areg[i] * 1024);
   };
-  auto load_s = [&](int grp) { buf_lds16(rs, soff, grp * 16, s.sa + (grp & 1) * 1024); };
+  auto load_s = [&](int grp) { buf_lds16(rs, soff, grp * 16, s.sa + (grp & 1) * kS + wave * 1024); };
 #pragma unroll
   for (int i = 0; i < NA; ++i) load_a(i, 0, 0);
-  if (wave == 0) {
+  if (wave < TR / 64) {
     load_s(0);
-    mid_st32(lds_addr(s.tok) + 4 * lane, ssrc);
+    mid_st32(lds_addr(s.tok) + 4 * srow, ssrc);
   }
   // weight block scales of the tile's two 128-row halves (gate / up, or two output blocks)
   for (int i = tid; i < 2 * KB; i += kMidThreads) {
@@ -232,15 +244,15 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
   const uint32_t sa_base = lds_addr(s.sa) + r16 * 16;
   const uint32_t w0_base = lds_addr(&s.sw[KIND == 0 ? 0 : wave >> 1][0]);
   const uint32_t w1_base = lds_addr(&s.sw[KIND == 0 ? 1 : wave >> 1][0]);
-  const uint32_t r_base = lds_addr(s.r) + 4 * r16 + (KIND == 1 ? 4 * kMidRows * (wave >> 1) : 0);
-  // Scale ratios: lane j of wave w owns row 32 (w % 2) + j % 32 of half w / 2 (the upper lanes
-  // repeat the lower ones) and writes block k + 1's during step k. Rows without a source
-  // use scale 1; a zero scale (an all-zero weight block, whose products are zero) repeats
-  // the previous one.
-  const int orow = 32 * (wave & 1) + (lane & 31), ohalf = wave >> 1;
+  const uint32_t r_base = lds_addr(s.r) + 4 * r16 + (KIND == 1 ? 4 * TR * (wave >> 1) : 0);
+  // Scale ratios: lane j of wave w owns row 64 (w % 2) + j of half w / 2 (of 64 rows: row
+  // 32 (w % 2) + j % 32, the upper lanes repeat the lower ones) and writes block k + 1's
+  // during step k. Rows without a source use scale 1; a zero scale (an all-zero weight block,
+  // whose products are zero) repeats the previous one.
+  const int orow = (TR / 2) * (wave & 1) + (lane & (TR / 2 - 1)), ohalf = wave >> 1;
   const uint32_t osa = lds_addr(s.sa) + 16 * orow;
   const uint32_t osw = lds_addr(&s.sw[ohalf][0]);
-  const uint32_t odst = lds_addr(s.r) + 4 * (kMidRows * ohalf + orow);
+  const uint32_t odst = lds_addr(s.r) + 4 * (TR * ohalf + orow);
   float s_prev = 0.f;
   bool ovalid = false;
   auto ratio = [&](float sa, float sw) {
@@ -259,7 +271,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     lds_barrier();  // ... for every wave, and its ratios are written
     v4i b[8];
     float nsa, nsw;
-    MidFragA f[2];
+    MidFragA f[D];
     constexpr int r1 = 16, r2 = KIND == 0 ? 128 : 32, r3 = KIND == 0 ? 144 : 48;
     mid_read16<0>(b_lo, b[0]);
     mid_read16<0>(b_hi, b[1]);
@@ -272,29 +284,30 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     // ratios: the next block's scales (past the last block: not used); otherwise this block's
     // weight scales of the wave's gate and up (or output) half
     if constexpr (RATIO) {
-      mid_read4<4 * ((Q + 1) & 3)>(osa + ((grp + (Q == 3)) & 1) * 1024, nsa);
+      mid_read4<4 * ((Q + 1) & 3)>(osa + ((grp + (Q == 3)) & 1) * kS, nsa);
       mid_read4<4 * (Q + 1)>(osw + 16 * grp, nsw);
     } else {
       mid_read4<4 * Q>(w0_base + 16 * grp, nsa);
       mid_read4<4 * Q>(w1_base + 16 * grp, nsw);
     }
-    const uint32_t ra0 = RATIO ? r_base : sa_base + (grp & 1) * 1024;
-    mid_read_a<KIND, BUF, Q, RATIO>(a_lo, a_hi, ra0, 0, f[0]);
+    const uint32_t ra0 = RATIO ? r_base : sa_base + (grp & 1) * kS;
+    mid_read_a<KIND, TR, BUF, Q, RATIO>(a_lo, a_hi, ra0, 0, f[0]);
     mid_wait_b<RATIO ? 4 : 3>(b, nsa, nsw);
     lds_barrier();  // every wave holds its weight fragments
     if (more) {
 #pragma unroll
       for (int i = 0; i < NA; ++i) load_a(i, kb + 1, BUF ^ 1);
       load_b(kb + 1);
-      if (Q == 0 && wave == 0) load_s(grp + 1);  // past the last group: not used
-      if constexpr (RATIO) mid_st32(odst + 8 * kMidRows * (BUF ^ 1), __float_as_int(ratio(nsa, nsw)));
+      if (Q == 0 && wave < TR / 64) load_s(grp + 1);  // past the last group: not used
+      if constexpr (RATIO) mid_st32(odst + 8 * TR * (BUF ^ 1), __float_as_int(ratio(nsa, nsw)));
     }
-    mid_wait<RATIO>(f[0]);
+    if (D > 2 && MF > 1) mid_read_a<KIND, TR, BUF, Q, RATIO>(a_lo, a_hi, ra0, 1, f[1]);
+    mid_wait<RATIO, (D > 2 && MF > 1) ? 4 : 0>(f[0]);
     if constexpr (!RATIO) {
       // fragment m's four products, scaled and added (the other workgroups' waves fill the wait)
 #pragma unroll
       for (int m = 0; m < MF; ++m) {
-        if (m + 1 < MF) mid_read_a<KIND, BUF, Q, RATIO>(a_lo, a_hi, ra0, m + 1, f[(m + 1) & 1]);
+        if (m + 1 < MF) mid_read_a<KIND, TR, BUF, Q, RATIO>(a_lo, a_hi, ra0, m + 1, f[(m + 1) & 1]);
         const v8i t = mid_cat(f[m & 1].lo, f[m & 1].hi);
         const float c0 = f[m & 1].r0 * nsa, c1 = f[m & 1].r0 * nsw;
         v4f part[4];
@@ -311,8 +324,8 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     }
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
-      if (m + 1 < MF) mid_read_a<KIND, BUF, Q, RATIO>(a_lo, a_hi, ra0, m + 1, f[(m + 1) & 1]);
-      const MidFragA& x = f[m & 1];
+      if (m + D - 1 < MF) mid_read_a<KIND, TR, BUF, Q, RATIO>(a_lo, a_hi, ra0, m + D - 1, f[(m + D - 1) % D]);
+      const MidFragA& x = f[m % D];
       const v8i t = mid_cat(x.lo, x.hi);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
@@ -321,7 +334,12 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
         __builtin_amdgcn_sched_barrier(0);
       }
       mid_pin(acc[m > 0 ? m - 1 : MF - 1]);
-      if (m + 1 < MF) mid_wait<RATIO>(f[(m + 1) & 1]);
+      if (m + 1 < MF) {
+        if (D > 2 && m + 2 < MF)
+          mid_wait<RATIO, 4>(f[(m + 1) % D]);
+        else
+          mid_wait<RATIO>(f[(m + 1) % D]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -349,7 +367,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
   __syncthreads();  // the last step's reads are done: its scale and ratio buffers are reused
   float* const last = (float*)s.sa;
   if constexpr (RATIO) {
-    last[kMidRows * ohalf + orow] = s_prev;
+    last[TR * ohalf + orow] = s_prev;
     __syncthreads();
   }
   // per-output-channel weight scales, 1 when absent (a multiply by 1 is exact)
@@ -369,7 +387,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     }
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
-      const float sg_ = RATIO ? last[16 * m + r16] : 1.f, su = RATIO ? last[kMidRows + 16 * m + r16] : 1.f;
+      const float sg_ = RATIO ? last[16 * m + r16] : 1.f, su = RATIO ? last[TR + 16 * m + r16] : 1.f;
       float mx = 0.f;
 #pragma unroll
       for (int n = 0; n < 2; ++n)
@@ -384,15 +402,15 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      if (g == 0) s.r[kMidRows * wave + 16 * m + r16] = mx;
+      if (g == 0) s.r[TR * wave + 16 * m + r16] = mx;
     }
     __syncthreads();
     const int GI = p.I / 128;
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
       const int row = 16 * m + r16;
-      const float amax = fmaxf(fmaxf(s.r[row], s.r[kMidRows + row]),
-                               fmaxf(s.r[2 * kMidRows + row], s.r[3 * kMidRows + row]));
+      const float amax = fmaxf(fmaxf(s.r[row], s.r[TR + row]),
+                               fmaxf(s.r[2 * TR + row], s.r[3 * TR + row]));
       const float sc = fmaxf(amax, 0x1.b7cdfep-34f) / 448.0f;
       const float rsc = 1.0f / sc;
       uint32_t c[2];
@@ -418,7 +436,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
       const int row = 16 * m + r16;
-      const float sl = RATIO ? last[kMidRows * (wave >> 1) + row] : 1.f;
+      const float sl = RATIO ? last[TR * (wave >> 1) + row] : 1.f;
       int o[8];
 #pragma unroll
       for (int n = 0; n < 4; ++n)
@@ -437,14 +455,14 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
 
 // RATIO: the block kernels' arithmetic on block tiles; otherwise the row-tile kernels' on row
 // tiles.
-template <int KIND, bool RATIO>
-__global__ __launch_bounds__(kMidThreads, 3) void expert_gemm_mid_kernel(MidArgs p) {
+template <int KIND, int TR, bool RATIO>
+__global__ __launch_bounds__(kMidThreads, TR > 64 ? 2 : 3) void expert_gemm_mid_kernel(MidArgs p) {
   __shared__ __attribute__((aligned(1024))) uint8_t sB[kMidCols * 128];
-  __shared__ __attribute__((aligned(1024))) uint8_t sA[2 * kMidA];
-  __shared__ __attribute__((aligned(1024))) uint8_t sSA[2 * kMidRows * 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t sA[2 * TR * 128];
+  __shared__ __attribute__((aligned(1024))) uint8_t sSA[2 * TR * 16];
   __shared__ float sW[2][kMidMaxKB];
-  __shared__ int sTok[kMidRows];
-  __shared__ float sR[4 * kMidRows];
+  __shared__ int sTok[TR];
+  __shared__ float sR[4 * TR];
   const MidLds s{sB, sA, sSA, sW, sTok, sR};
   const int NT = (KIND == 0) ? p.I / 128 : p.H / kMidCols;
   int tile, nt;
@@ -473,13 +491,23 @@ __global__ __launch_bounds__(kMidThreads, 3) void expert_gemm_mid_kernel(MidArgs
   const int4 td = make_int4(__builtin_amdgcn_readfirstlane(tv.x), __builtin_amdgcn_readfirstlane(tv.y),
                             __builtin_amdgcn_readfirstlane(tv.z), __builtin_amdgcn_readfirstlane(tv.w));
   const int e = td.x, nrows = td.z;
-  if (e < 0 || e >= p.E + p.nsh || nrows <= 0 || nrows > kMidRows) return;
-  switch ((nrows + 15) / 16) {
-    case 1: return mid_item<KIND, 1, RATIO>(p, s, e, td.y, td.w, nrows, nt, alone);
-    case 2: return mid_item<KIND, 2, RATIO>(p, s, e, td.y, td.w, nrows, nt, alone);
-    case 3: return mid_item<KIND, 3, RATIO>(p, s, e, td.y, td.w, nrows, nt, alone);
-    default: return mid_item<KIND, 4, RATIO>(p, s, e, td.y, td.w, nrows, nt, alone);
+  if (e < 0 || e >= p.E + p.nsh || nrows <= 0 || nrows > TR) return;
+#define MID_ITEM(MF) return mid_item<KIND, TR, MF, RATIO>(p, s, e, td.y, td.w, nrows, nt, alone)
+  if constexpr (TR > 64) {
+    switch ((nrows + 15) / 16) {
+      case 5: MID_ITEM(5);
+      case 6: MID_ITEM(6);
+      case 7: MID_ITEM(7);
+      case 8: MID_ITEM(8);
+    }
   }
+  switch ((nrows + 15) / 16) {
+    case 1: MID_ITEM(1);
+    case 2: MID_ITEM(2);
+    case 3: MID_ITEM(3);
+    default: MID_ITEM(4);
+  }
+#undef MID_ITEM
 }
 
 bool mid_fits(int kind, const MidArgs& a) {
@@ -491,30 +519,31 @@ bool mid_fits(int kind, const MidArgs& a) {
          2UL * a.I * a.H < lim && a.rows < (1L << 31);
 }
 
-void launch_mid(int kind, const MidArgs& a, int max_tiles, hipStream_t st) {
-  const long NT = (kind == 0) ? a.I / 128 : a.H / kMidCols;
-  // block tiles: each XCD's share of them
-  const long items = (a.seg != nullptr ? 8L * block_tiles_cap(max_tiles) : (long)max_tiles) * NT;
+template <int TR, bool RATIO>
+static void launch_mid_tiles(int kind, const MidArgs& a, long items, hipStream_t st) {
   const dim3 grid((unsigned)items), block(kMidThreads);
-  if (kind == 0) {
-    if (a.seg != nullptr)
-      hipLaunchKernelGGL((expert_gemm_mid_kernel<0, true>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((expert_gemm_mid_kernel<0, false>), grid, block, 0, st, a);
-  } else {
-    if (a.seg != nullptr)
-      hipLaunchKernelGGL((expert_gemm_mid_kernel<1, true>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((expert_gemm_mid_kernel<1, false>), grid, block, 0, st, a);
-  }
+  if (kind == 0)
+    hipLaunchKernelGGL((expert_gemm_mid_kernel<0, TR, RATIO>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((expert_gemm_mid_kernel<1, TR, RATIO>), grid, block, 0, st, a);
+}
+
+void launch_mid(int kind, const MidArgs& a, int max_tiles, int rows, hipStream_t st) {
+  const long NT = (kind == 0) ? a.I / 128 : a.H / kMidCols;
+  if (a.seg == nullptr) return launch_mid_tiles<kMidTileRows, false>(kind, a, (long)max_tiles * NT, st);
+  const long items = 8L * block_tiles_cap(max_tiles) * NT;  // each XCD's share of the block tiles
+  if (rows > kMidTileRows)
+    launch_mid_tiles<kMidTallRows, true>(kind, a, items, st);
+  else
+    launch_mid_tiles<kMidTileRows, true>(kind, a, items, st);
 }
 
 }  // namespace moe
 
 using namespace moe;
 
-int moe::mid_max_tiles(int T, int K, int E, int n_shared) {
+int moe::mid_max_tiles(int T, int K, int E, int n_shared, int tile_rows) {
   const long rows = (long)T * std::min(K, E);
-  return (int)(rows / kMidTileRows + std::min<long>(E, rows) +
-               (long)n_shared * ((T + kMidTileRows - 1) / kMidTileRows));
+  return (int)(rows / tile_rows + std::min<long>(E, rows) +
+               (long)n_shared * ((T + tile_rows - 1) / tile_rows));
 }

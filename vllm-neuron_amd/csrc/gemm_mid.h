@@ -33,7 +33,7 @@ struct MidArgs {
 // and operands that 32-bit byte offsets reach. Otherwise the other kernels run.
 bool mid_fits(int kind, const MidArgs& a);
 // Launch on a.tiles: block tiles (a.seg set, XCD ranges in the header num_tiles) or row tiles,
-// of at most kMidTileRows rows.
-void launch_mid(int kind, const MidArgs& a, int max_tiles, hipStream_t st);
+// of at most `rows` rows: kMidTileRows, or for block tiles kMidTallRows.
+void launch_mid(int kind, const MidArgs& a, int max_tiles, int rows, hipStream_t st);
 
 }  // namespace moe

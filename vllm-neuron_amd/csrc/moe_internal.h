@@ -29,12 +29,19 @@ constexpr int kBlockTileRows = 256;
 constexpr int kMxBlockTileRows = 128;
 
 // Rows per tile of the mid-size fp8 expert GEMM kernels (gemm_fp8_mid.hip). The layer runs
-// them instead of the block kernels from 32 up to kMidMaxRows routed rows per expert on
-// average: layer, block -> mid-size kernels, at 33 rows DeepSeek-V3 2127 -> 2020 us and Kimi-K2
+// them instead of the block kernels from 32 routed rows per expert on average: 64-row tiles up
+// to kMidMaxRows, 128-row tiles up to kMidTallMaxRows.
+// Layer, block -> 64-row kernels, at 33 rows DeepSeek-V3 2127 -> 2020 us and Kimi-K2
 // 3134 -> 3051 us, at 35 GLM-4.5 805 -> 741 us; at 41 DeepSeek-V3 2165 -> 2158 us; at 50 and
 // above, where experts take two 64-row tiles, they lose (DeepSeek-V3 2241 -> 2294 us).
+// Block -> 128-row kernels: at 42 rows Kimi-K2 3228 -> 3132 and GLM-4.5 827 -> 803 us, at 75
+// DeepSeek-V3 2405 -> 2365, Kimi-K2 3613 -> 3584 and GLM-4.5 920 -> 863 us; at 81 and 83
+// DeepSeek-V3 2462 -> 2486 and Kimi-K2 3688 -> 3692 us (GLM-4.5 gains up to 115), at 125 to 256
+// the block kernels lead by up to 4 % (two thirds of the global -> LDS bytes per product).
 constexpr int kMidTileRows = 64;
+constexpr int kMidTallRows = 128;
 constexpr int kMidMaxRows = 40;
+constexpr int kMidTallMaxRows = 76;
 // Work items (two per CU) from which they run 16-row tiles and small layers.
 constexpr long kMidMinItems = 512;
 
@@ -162,8 +169,8 @@ int layer_down_combine_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, in
                           const int32_t* ids, const int32_t* inv, const float* weights,
                           void* out_bf16, void* stream, bool* done);
 
-// Most block tiles of kMidTileRows rows that the layer's mapping writes (compact rows).
-int mid_max_tiles(int T, int K, int E, int n_shared);
+// Most block tiles of tile_rows rows that the layer's mapping writes (compact rows).
+int mid_max_tiles(int T, int K, int E, int n_shared, int tile_rows);
 
 // Most block tiles of kMxBlockTileRows rows that the layer's mapping writes (compact rows).
 int mx_block_max_tiles(int T, int K, int E);
