@@ -228,6 +228,30 @@ int moe_expert_down_block(const uint8_t* hq, const float* hs, int T, int H, int 
                           const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
                           void* y_bf16, void* stream);
 
+/* The same on tiles of at most tile_rows rows, 128 or 256 (the functions above: 256), which all
+ * four calls get alike. With 128 the GEMMs run kernels with two workgroups per CU where they
+ * can (H and I multiples of 512, no channel scales): faster up to about 76 rows per expert. */
+int moe_max_block_tiles_rows(int T, int K, int E, int N, int B, int n_shared, int tile_rows);
+int moe_build_block_tiles_rows(const int32_t* token_position_to_id, const int32_t* block_to_expert,
+                               int N, int B, int T, int E, int n_shared, int tile_rows,
+                               int32_t* tiles, int max_tiles, int32_t* num_tiles, void* workspace,
+                               size_t workspace_bytes, void* stream);
+int moe_expert_gate_up_block_rows(const uint8_t* xq, const float* xs, int T, int H, int I, int E,
+                                  const uint8_t* w13, const float* w13_scale,
+                                  const float* w13_channel_scale, const uint8_t* w13_shared,
+                                  const float* w13_shared_scale,
+                                  const float* w13_shared_channel_scale, int n_shared,
+                                  const int32_t* token_position_to_id, int NB,
+                                  const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
+                                  int tile_rows, uint8_t* hq, float* hs, void* stream);
+int moe_expert_down_block_rows(const uint8_t* hq, const float* hs, int T, int H, int I, int E,
+                               const uint8_t* w2, const float* w2_scale,
+                               const float* w2_channel_scale, const uint8_t* w2_shared,
+                               const float* w2_shared_scale,
+                               const float* w2_shared_channel_scale, int n_shared, int NB,
+                               const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
+                               int tile_rows, void* y_bf16, void* stream);
+
 /* ---- weighted unpermute-combine ----------------------------------------- */
 
 /* out[t] = bf16( sum_{s<S, inv[t,s]>=0} w[t,s] * y[inv[t,s]]  +  sum_{j<n_shared} y[NB + j*T + t] ),

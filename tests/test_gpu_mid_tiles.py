@@ -104,3 +104,38 @@ def test_layer_block_tiles_equal_block_kernels(cuda, T, S, zero):
     y = ops.expert_down_block(hq, hs, w, T, NB, tiles, num, mx)
     ref = ops.combine(y, m["inv_pos"], wts, T, H, NB, S)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+# The operators' block tile lists of up to 128 rows against those of up to 256 on the block
+# kernels, whose rows' results do not depend on the tile. The last two cases (H not a multiple of 512,
+# channel scales) run the block kernels on both.
+@pytest.mark.parametrize("H,I,S,chan", [(512, 512, 0, False), (1024, 1536, 1, False), (2560, 512, 2, False),
+                                        (768, 512, 0, False), (512, 512, 1, True)])
+def test_tall_tile_lists_equal_block_lists(cuda, H, I, S, chan):
+    counts = [1, 16, 17, 0, 33, 64, 65, 81, 97, 112, 113, 127, 128, 129, 256, 257, 300]
+    E, T = len(counts), sum(counts)
+    say("tall tile lists", H, I, S, chan, T)
+    w = synthetic.make_weights(MoEConfig(H, I, E, 1, n_shared=S), 7, device=cuda)
+    if chan:
+        g = torch.Generator(device=cuda).manual_seed(9)
+        c = lambda *s: torch.rand(*s, device=cuda, generator=g) + 0.5
+        w = dataclasses.replace(w, w13_chan=c(E, 2 * I), w2_chan=c(E, H), shared_w13_chan=c(S, 2 * I),
+                                shared_w2_chan=c(S, H))
+    ids = torch.from_numpy(np.random.default_rng(1).permutation(np.repeat(np.arange(E), counts))
+                           .astype(np.int32).reshape(T, 1)).to(cuda)
+    m = ops.blockwise_mapping(ids=ids, n_experts=E, block_size=64)
+    tpid, b2e = m["token_position_to_id"].clone(), m["block_to_expert"]
+    tpid[(tpid >= 0).nonzero()[5]] = -1  # a hole inside a tile: its h row is not written
+    xq, xs = ops.act_quant(synthetic.hidden_states(T, H, 7).to(cuda))
+    live = torch.cat([tpid >= 0, torch.ones(S * T, dtype=torch.bool, device=cuda)])
+    got = []
+    for rows in (128, 256):
+        tiles, num, mx = ops.build_block_tiles(tpid, b2e, 64, T, 1, E, S, rows)
+        hq, hs = ops.expert_gate_up_block(xq, xs, w, tpid, tpid.numel(), tiles, num, mx, rows)
+        y = ops.expert_down_block(hq, hs, w, T, tpid.numel(), tiles, num, mx, rows)
+        n = int(num[0])
+        got.append((hq[live].view(torch.uint8), hs[live], y[live].view(torch.int16)))
+        assert n <= mx and int(tiles[: 4 * n].view(n, 4)[:, 2].max()) <= rows
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert float(y[live].float().abs().max()) > 0

@@ -39,6 +39,7 @@
 // Fragment lane layout (16x16x128): lane l supplies row l%16 and the bytes
 // [(l/16)*16, +16) and [64 + (l/16)*16, +16) of the 128-wide K block, the same
 // mapping for A and B. Accumulator: lane l, register i holds D[4*(l/16) + i][l%16].
+#include "gemm_mid.h"
 #include "mapping.h"
 #include "moe_common.h"
 #include "moe_internal.h"
@@ -650,9 +651,9 @@ __global__ __launch_bounds__(kBlkThreads) void expert_gemm_block_kernel(BlkArgs 
 
 // ---------------------------------------------------------------------------
 // Block tiles: per expert segment (consecutive blocks with one expert id), the
-// slot range from its first block to its last valid slot, cut into chunks of
-// 256 rows; seg[t] = {first tile of the segment, tiles in the segment}.
-// Shared experts j: ceil(T/256) tiles over slots [NB + j*T, NB + (j+1)*T).
+// slot range from its first block to its last valid slot, cut into chunks of at most
+// mt (256 or 128) rows; seg[t] = {first tile of the segment, tiles in the segment}.
+// Shared experts j: ceil(T/mt) tiles over slots [NB + j*T, NB + (j+1)*T).
 // num_tiles[0] = the tile count, num_tiles[1..9] = the XCD ranges.
 // One workgroup; per-block last-valid lengths go through LDS, or global scratch past
 // kSegLds blocks.
@@ -664,7 +665,7 @@ constexpr int kSegLds = 2048;
 
 __global__ __launch_bounds__(1024) void build_block_tiles_kernel(
     const int32_t* __restrict__ tpid, const int32_t* __restrict__ b2e, int N, int B, int T, int E,
-    int n_shared, int* __restrict__ vlen, int4* __restrict__ tiles,
+    int n_shared, int mt, int* __restrict__ vlen, int4* __restrict__ tiles,
     int2* __restrict__ seg, int max_tiles, int32_t* __restrict__ num_tiles) {
   __shared__ int s_e[kSegLds], s_v[kSegLds];
   __shared__ int s_first[kSegLds], s_cost[kSegLds];  // per non-empty segment: first tile, cost before it
@@ -731,7 +732,7 @@ __global__ __launch_bounds__(1024) void build_block_tiles_kernel(
       if (last >= 0) {
         s0 = (long)b * B;
         s1 = (long)last * B + len(last);
-        v = (int)((s1 - s0 + kBM - 1) / kBM);
+        v = (int)((s1 - s0 + mt - 1) / mt);
       }
     }
     const long h = v > 0 ? (s1 - s0 + v - 1) / v : 0;  // equal heights (sibling tiles share weight blocks in L2)
@@ -766,7 +767,7 @@ __global__ __launch_bounds__(1024) void build_block_tiles_kernel(
     cost += s_chunk[2];
     __syncthreads();
   }
-  const int per = (T + kBM - 1) / kBM;
+  const int per = (T + mt - 1) / mt;
   const int hsh = (T + per - 1) / per;
   const long NB = (long)N * B;
   for (int i = tid; i < n_shared * per; i += blockDim.x) {
@@ -805,10 +806,16 @@ static void launch_block(const BlkArgs& a, int max_tiles, hipStream_t st) {
 
 using namespace moe;
 
+static bool block_rows_ok(int tile_rows) { return tile_rows == kBM || tile_rows == kMidTallRows; }
+
+extern "C" int moe_max_block_tiles_rows(int T, int K, int E, int N, int B, int n_shared, int tile_rows) {
+  if (T <= 0 || K <= 0 || E <= 0 || N <= 0 || B <= 0 || n_shared < 0 || !block_rows_ok(tile_rows)) return 0;
+  const long routed = ((long)N * B + tile_rows - 1) / tile_rows + std::min(E, N);
+  return (int)(routed + (long)n_shared * ((T + tile_rows - 1) / tile_rows));
+}
+
 extern "C" int moe_max_block_tiles(int T, int K, int E, int N, int B, int n_shared) {
-  if (T <= 0 || K <= 0 || E <= 0 || N <= 0 || B <= 0 || n_shared < 0) return 0;
-  const long routed = ((long)N * B + kBM - 1) / kBM + std::min(E, N);
-  return (int)(routed + (long)n_shared * ((T + kBM - 1) / kBM));
+  return moe_max_block_tiles_rows(T, K, E, N, B, n_shared, kBM);
 }
 
 extern "C" size_t moe_block_tiles_workspace_bytes(int N, int max_tiles) {
@@ -816,12 +823,12 @@ extern "C" size_t moe_block_tiles_workspace_bytes(int N, int max_tiles) {
   return (size_t)N * 8 + (size_t)max_tiles * 24 + 256;
 }
 
-extern "C" int moe_build_block_tiles(const int32_t* token_position_to_id,
+static int build_block_tiles(const char* _moe_fn, const int32_t* token_position_to_id,
                                      const int32_t* block_to_expert, int N, int B, int T, int E,
-                                     int n_shared, int32_t* tiles, int max_tiles,
+                                     int n_shared, int tile_rows, int32_t* tiles, int max_tiles,
                                      int32_t* num_tiles, void* workspace, size_t workspace_bytes,
                                      void* stream) {
-  MOE_API_BEGIN("moe_build_block_tiles");
+  MOE_CHECK_ARG(block_rows_ok(tile_rows), "tile_rows must be 128 or 256, not %d", tile_rows);
   MOE_CHECK_ARG(token_position_to_id && block_to_expert && tiles && num_tiles && workspace,
                 "null pointer argument");
   MOE_CHECK_ARG(N > 0 && B > 0 && T > 0 && E > 0 && n_shared >= 0 && max_tiles > 0, "bad sizes");
@@ -830,9 +837,59 @@ extern "C" int moe_build_block_tiles(const int32_t* token_position_to_id,
   // tiles buffer holds int4 tiles followed by int2 segments: max_tiles * 24 bytes
   int* vlen = (int*)workspace;
   hipLaunchKernelGGL(build_block_tiles_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream,
-                     token_position_to_id, block_to_expert, N, B, T, E, n_shared, vlen,
+                     token_position_to_id, block_to_expert, N, B, T, E, n_shared, tile_rows, vlen,
                      (int4*)tiles, (int2*)(tiles + 4 * (size_t)max_tiles), max_tiles, num_tiles);
   MOE_API_END();
+}
+
+extern "C" int moe_build_block_tiles(const int32_t* token_position_to_id,
+                                     const int32_t* block_to_expert, int N, int B, int T, int E, int n_shared, int32_t* tiles,
+                                     int max_tiles, int32_t* num_tiles, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  MOE_API_BEGIN("moe_build_block_tiles");
+  return build_block_tiles(_moe_fn, token_position_to_id, block_to_expert, N, B, T, E, n_shared, kBM,
+                           tiles, max_tiles, num_tiles, workspace, workspace_bytes, stream);
+}
+
+extern "C" int moe_build_block_tiles_rows(const int32_t* token_position_to_id,
+                                          const int32_t* block_to_expert, int N, int B, int T, int E,
+                                          int n_shared, int tile_rows, int32_t* tiles, int max_tiles,
+                                          int32_t* num_tiles, void* workspace, size_t workspace_bytes,
+                                          void* stream) {
+  MOE_API_BEGIN("moe_build_block_tiles_rows");
+  return build_block_tiles(_moe_fn, token_position_to_id, block_to_expert, N, B, T, E, n_shared, tile_rows,
+                           tiles, max_tiles, num_tiles, workspace, workspace_bytes, stream);
+}
+
+// On tiles of up to kMidTallRows rows the mid-size kernels run where they can (whole K groups,
+// no per-channel scales); this file's kernels take any tile.
+template <int KIND>
+static void launch_block_rows(const BlkArgs& a, int tile_rows, int max_tiles, hipStream_t st) {
+  MidArgs m{};
+  m.a = a.a;
+  m.as = a.as;
+  m.w = a.w;
+  m.ws = a.ws;
+  m.wsh = a.wsh;
+  m.wssh = a.wssh;
+  m.tpid = a.tpid;
+  m.tiles = a.tiles;
+  m.seg = a.seg;
+  m.num_tiles = a.num_tiles;
+  m.hq = a.hq;
+  m.hs = a.hs;
+  m.y = a.y;
+  m.T = a.T;
+  m.H = a.H;
+  m.I = a.I;
+  m.E = a.E;
+  m.nsh = a.nsh;
+  m.NB = a.NB;
+  m.rows = a.NB + (long)a.nsh * a.T;
+  if (tile_rows == kMidTallRows && a.cs == nullptr && a.cssh == nullptr && mid_fits(KIND, m))
+    launch_mid(KIND, m, max_tiles, kMidTallRows, st);
+  else
+    launch_block<KIND>(a, max_tiles, st);
 }
 
 // a_rows x a_cols: the gathered operand (x for gate_up, h for down), addressed with
@@ -849,15 +906,14 @@ static int block_gemm_common_checks(const char* _moe_fn, int T, int H, int I, in
   return MOE_OK;
 }
 
-extern "C" int moe_expert_gate_up_block(const uint8_t* xq, const float* xs, int T, int H, int I,
-                                        int E, const uint8_t* w13, const float* w13_scale,
-                                        const float* w13_channel_scale, const uint8_t* w13_shared,
-                                        const float* w13_shared_scale,
-                                        const float* w13_shared_channel_scale, int n_shared,
-                                        const int32_t* token_position_to_id, int NB,
-                                        const int32_t* tiles, const int32_t* num_tiles,
-                                        int max_tiles, uint8_t* hq, float* hs, void* stream) {
-  MOE_API_BEGIN("moe_expert_gate_up_block");
+static int expert_gate_up_block(const char* _moe_fn, const uint8_t* xq, const float* xs, int T, int H,
+                                int I, int E, const uint8_t* w13, const float* w13_scale,
+                                const float* w13_channel_scale, const uint8_t* w13_shared,
+                                const float* w13_shared_scale, const float* w13_shared_channel_scale,
+                                int n_shared, const int32_t* token_position_to_id, int NB,
+                                const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
+                                uint8_t* hq, float* hs, void* stream, int tile_rows) {
+  MOE_CHECK_ARG(block_rows_ok(tile_rows), "tile_rows must be 128 or 256, not %d", tile_rows);
   MOE_CHECK_ARG(xq && xs && w13 && w13_scale && token_position_to_id && tiles && num_tiles && hq && hs,
                 "null pointer argument");
   int rc = block_gemm_common_checks(_moe_fn, T, H, I, E, NB, max_tiles, T, H);
@@ -886,19 +942,47 @@ extern "C" int moe_expert_gate_up_block(const uint8_t* xq, const float* xs, int 
   a.E = E;
   a.nsh = n_shared;
   a.NB = NB;
-  launch_block<0>(a, max_tiles, (hipStream_t)stream);
+  launch_block_rows<0>(a, tile_rows, max_tiles, (hipStream_t)stream);
   MOE_API_END();
 }
 
-extern "C" int moe_expert_down_block(const uint8_t* hq, const float* hs, int T, int H, int I, int E,
-                                     const uint8_t* w2, const float* w2_scale,
-                                     const float* w2_channel_scale, const uint8_t* w2_shared,
-                                     const float* w2_shared_scale,
-                                     const float* w2_shared_channel_scale, int n_shared, int NB,
-                                     const int32_t* tiles,
-                                     const int32_t* num_tiles, int max_tiles, void* y_bf16,
-                                     void* stream) {
-  MOE_API_BEGIN("moe_expert_down_block");
+extern "C" int moe_expert_gate_up_block(const uint8_t* xq, const float* xs, int T, int H, int I, int E,
+                                        const uint8_t* w13, const float* w13_scale,
+                                        const float* w13_channel_scale, const uint8_t* w13_shared,
+                                        const float* w13_shared_scale,
+                                        const float* w13_shared_channel_scale, int n_shared,
+                                        const int32_t* token_position_to_id, int NB,
+                                        const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
+                                        uint8_t* hq, float* hs, void* stream) {
+  MOE_API_BEGIN("moe_expert_gate_up_block");
+  return expert_gate_up_block(_moe_fn, xq, xs, T, H, I, E, w13, w13_scale, w13_channel_scale,
+                              w13_shared, w13_shared_scale, w13_shared_channel_scale, n_shared,
+                              token_position_to_id, NB, tiles, num_tiles, max_tiles, hq, hs, stream, kBM);
+}
+
+extern "C" int moe_expert_gate_up_block_rows(const uint8_t* xq, const float* xs, int T, int H, int I,
+                                             int E, const uint8_t* w13, const float* w13_scale,
+                                             const float* w13_channel_scale, const uint8_t* w13_shared,
+                                             const float* w13_shared_scale,
+                                             const float* w13_shared_channel_scale, int n_shared,
+                                             const int32_t* token_position_to_id, int NB,
+                                             const int32_t* tiles, const int32_t* num_tiles,
+                                             int max_tiles, int tile_rows, uint8_t* hq, float* hs,
+                                             void* stream) {
+  MOE_API_BEGIN("moe_expert_gate_up_block_rows");
+  return expert_gate_up_block(_moe_fn, xq, xs, T, H, I, E, w13, w13_scale, w13_channel_scale,
+                              w13_shared, w13_shared_scale, w13_shared_channel_scale, n_shared,
+                              token_position_to_id, NB, tiles, num_tiles, max_tiles, hq, hs, stream,
+                              tile_rows);
+}
+
+static int expert_down_block(const char* _moe_fn, const uint8_t* hq, const float* hs, int T, int H,
+                             int I, int E, const uint8_t* w2, const float* w2_scale,
+                             const float* w2_channel_scale, const uint8_t* w2_shared,
+                             const float* w2_shared_scale, const float* w2_shared_channel_scale,
+                             int n_shared, int NB, const int32_t* tiles, const int32_t* num_tiles,
+                             int max_tiles, void* y_bf16, void* stream, int tile_rows) {
+  MOE_CHECK_ARG(block_rows_ok(tile_rows), "tile_rows must be 128 or 256, not %d", tile_rows);
   MOE_CHECK_ARG(hq && hs && w2 && w2_scale && tiles && num_tiles && y_bf16, "null pointer argument");
   int rc = block_gemm_common_checks(_moe_fn, T, H, I, E, NB, max_tiles,
                                     (long)NB + (long)n_shared * T, I);
@@ -925,6 +1009,31 @@ extern "C" int moe_expert_down_block(const uint8_t* hq, const float* hs, int T, 
   a.E = E;
   a.nsh = n_shared;
   a.NB = NB;
-  launch_block<1>(a, max_tiles, (hipStream_t)stream);
+  launch_block_rows<1>(a, tile_rows, max_tiles, (hipStream_t)stream);
   MOE_API_END();
+}
+
+extern "C" int moe_expert_down_block(const uint8_t* hq, const float* hs, int T, int H, int I, int E,
+                                     const uint8_t* w2, const float* w2_scale,
+                                     const float* w2_channel_scale, const uint8_t* w2_shared,
+                                     const float* w2_shared_scale, const float* w2_shared_channel_scale,
+                                     int n_shared, int NB, const int32_t* tiles,
+                                     const int32_t* num_tiles, int max_tiles, void* y_bf16, void* stream) {
+  MOE_API_BEGIN("moe_expert_down_block");
+  return expert_down_block(_moe_fn, hq, hs, T, H, I, E, w2, w2_scale, w2_channel_scale, w2_shared,
+                           w2_shared_scale, w2_shared_channel_scale, n_shared, NB, tiles, num_tiles,
+                           max_tiles, y_bf16, stream, kBM);
+}
+
+extern "C" int moe_expert_down_block_rows(const uint8_t* hq, const float* hs, int T, int H, int I,
+                                          int E, const uint8_t* w2, const float* w2_scale,
+                                          const float* w2_channel_scale, const uint8_t* w2_shared,
+                                          const float* w2_shared_scale,
+                                          const float* w2_shared_channel_scale, int n_shared, int NB,
+                                          const int32_t* tiles, const int32_t* num_tiles, int max_tiles,
+                                          int tile_rows, void* y_bf16, void* stream) {
+  MOE_API_BEGIN("moe_expert_down_block_rows");
+  return expert_down_block(_moe_fn, hq, hs, T, H, I, E, w2, w2_scale, w2_channel_scale, w2_shared,
+                           w2_shared_scale, w2_shared_channel_scale, n_shared, NB, tiles, num_tiles,
+                           max_tiles, y_bf16, stream, tile_rows);
 }

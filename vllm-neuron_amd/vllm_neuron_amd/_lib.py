@@ -59,6 +59,12 @@ PROTOTYPES = {
                                       _p, _p, _i, _p, _p, _p]),
     "moe_expert_down_block": (_i, [_p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p,
                                    _i, _p, _p]),
+    "moe_max_block_tiles_rows": (_i, [_i, _i, _i, _i, _i, _i, _i]),
+    "moe_build_block_tiles_rows": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _sz, _p]),
+    "moe_expert_gate_up_block_rows": (_i, [_p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p,
+                                           _i, _p, _p, _i, _i, _p, _p, _p]),
+    "moe_expert_down_block_rows": (_i, [_p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _i, _p,
+                                        _p, _i, _i, _p, _p]),
     "moe_act_quant_mx": (_i, [_p, _i, _i, _p, _p, _p]),
     "moe_expert_gate_up_mx": (_i, [_p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p, _i,
                                    _p, _p, _i, _i, _i, _f, _f, _f, _f, _p, _p, _p]),

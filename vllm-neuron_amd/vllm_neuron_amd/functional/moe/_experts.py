@@ -261,9 +261,10 @@ def run_experts(x_bf16, tpid, b2e, B, k_rows, k_bound, w, xq=None, xs=None):
     if xq is None:
         xq, xs = ops.act_quant(x_bf16)
     if ops.use_block_kernels(T, k_rows, E):
-        tiles, num, mbt = ops.build_block_tiles(tpid, b2e, B, T, k_bound, E, S)
-        hq, hs = ops.expert_gate_up_block(xq, xs, w, tpid, NB, tiles, num, mbt)
-        y = ops.expert_down_block(hq, hs, w, T, NB, tiles, num, mbt)
+        rows = ops.block_tile_rows(T, k_rows, E, w)
+        tiles, num, mbt = ops.build_block_tiles(tpid, b2e, B, T, k_bound, E, S, rows)
+        hq, hs = ops.expert_gate_up_block(xq, xs, w, tpid, NB, tiles, num, mbt, rows)
+        y = ops.expert_down_block(hq, hs, w, T, NB, tiles, num, mbt, rows)
     else:
         mt = ops.choose_mt(T, k_rows, E)
         tiles, num, max_tiles = ops.build_tiles(tpid, b2e, B, T, k_bound, E, S, mt)

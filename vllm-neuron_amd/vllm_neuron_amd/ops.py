@@ -51,6 +51,16 @@ def use_block_kernels(T, K, E):
     return -(-T * min(K, E) // E) > 32
 
 
+def block_tile_rows(T, K, E, w):
+    """Rows per tile of the block tile lists for weights w: 128 (kernels with two workgroups per
+    CU) up to 76 rows per expert on average, the layer's bound, where the weights suit them
+    and fill the chip; else 256."""
+    H, I = w.hidden, w.w13.shape[1] // 2
+    tall = (T * min(K, E) <= 76 * E and H % 512 == 0 and I % 512 == 0
+            and not w.has_channel_scales and E * (I // 128) >= 512)
+    return 128 if tall else 256
+
+
 def choose_mt(T, K, E):
     avg = -(-T * min(K, E) // E)
     for limit, mt in ((4, 16), (24, 32), (48, 64)):
@@ -288,45 +298,46 @@ def combine(y, inv, wts, T, H, NB, n_shared):
     return out
 
 
-def build_block_tiles(tpid, b2e, B, T, K, E, n_shared):
-    """Tile list of the prefill-sized kernels (up to 256 slots of one expert per tile)."""
+def build_block_tiles(tpid, b2e, B, T, K, E, n_shared, tile_rows=256):
+    """Tile list of the prefill-sized kernels (up to tile_rows, 256 or 128, slots of one expert
+    per tile)."""
     N = b2e.numel()
     lib = _lib.load()
-    max_tiles = lib.moe_max_block_tiles(T, K, E, N, B, n_shared)
+    max_tiles = lib.moe_max_block_tiles_rows(T, K, E, N, B, n_shared, tile_rows)
     tiles = torch.empty(max_tiles * 6, device=tpid.device, dtype=torch.int32)
     # the list's header: the tile count, then the XCD ranges the block kernels read
     num = torch.empty(BLOCK_TILES_HEADER, device=tpid.device, dtype=torch.int32)
     wsb = lib.moe_block_tiles_workspace_bytes(N, max_tiles)
     ws = torch.empty(wsb, device=tpid.device, dtype=torch.uint8)
-    _lib.call("moe_build_block_tiles", ptr(tpid), ptr(b2e), N, B, T, E, n_shared, ptr(tiles),
-              max_tiles, ptr(num), ptr(ws), wsb, _stream())
+    _lib.call("moe_build_block_tiles_rows", ptr(tpid), ptr(b2e), N, B, T, E, n_shared, tile_rows,
+              ptr(tiles), max_tiles, ptr(num), ptr(ws), wsb, _stream())
     return tiles, num, max_tiles
 
 
-def expert_gate_up_block(xq, xs, w, tpid, NB, tiles, num_tiles, max_tiles):
+def expert_gate_up_block(xq, xs, w, tpid, NB, tiles, num_tiles, max_tiles, tile_rows=256):
     T, H = xq.shape
     E, I2, _ = w.w13.shape
     I = I2 // 2
     S = w.n_shared
     hq = torch.empty(NB + S * T, I, device=xq.device, dtype=FP8)
     hs = torch.empty(NB + S * T, I // 128, device=xq.device, dtype=torch.float32)
-    _lib.call("moe_expert_gate_up_block", ptr(_u8(xq)), ptr(xs), T, H, I, E, ptr(_u8(w.w13)),
+    _lib.call("moe_expert_gate_up_block_rows", ptr(_u8(xq)), ptr(xs), T, H, I, E, ptr(_u8(w.w13)),
               ptr(w.w13_scale), ptr(w.w13_chan), ptr(_u8(w.shared_w13)) if S else None,
               ptr(w.shared_w13_scale) if S else None, ptr(w.shared_w13_chan) if S else None, S,
               ptr(tpid), NB, ptr(tiles),
-              ptr(num_tiles), max_tiles, ptr(_u8(hq)), ptr(hs), _stream())
+              ptr(num_tiles), max_tiles, tile_rows, ptr(_u8(hq)), ptr(hs), _stream())
     return hq, hs
 
 
-def expert_down_block(hq, hs, w, T, NB, tiles, num_tiles, max_tiles):
+def expert_down_block(hq, hs, w, T, NB, tiles, num_tiles, max_tiles, tile_rows=256):
     E, H, I = w.w2.shape
     S = w.n_shared
     y = torch.empty(hq.shape[0], H, device=hq.device, dtype=torch.bfloat16)
-    _lib.call("moe_expert_down_block", ptr(_u8(hq)), ptr(hs), T, H, I, E, ptr(_u8(w.w2)),
+    _lib.call("moe_expert_down_block_rows", ptr(_u8(hq)), ptr(hs), T, H, I, E, ptr(_u8(w.w2)),
               ptr(w.w2_scale), ptr(w.w2_chan), ptr(_u8(w.shared_w2)) if S else None,
               ptr(w.shared_w2_scale) if S else None, ptr(w.shared_w2_chan) if S else None, S, NB,
               ptr(tiles), ptr(num_tiles),
-              max_tiles, ptr(y), _stream())
+              max_tiles, tile_rows, ptr(y), _stream())
     return y
 
 
