@@ -167,6 +167,23 @@ def test_router_api(cuda, order, activation, with_gamma):
         assert np.allclose(a, ref, rtol=1e-6, atol=0)
 
 
+# bf16 operands under the fp32 computation dtype take the bf16 matrix cores: the fp32 product's
+# bound (test_router_logits_f32), also for rows that start off a 16-byte boundary.
+@pytest.mark.parametrize("T,H,E,offset", [(1, 64, 5, 0), (65, 512, 24, 1), (130, 2880, 128, 4), (2049, 1024, 160, 8)])
+def test_router_bf16_operands_fp32_logits(cuda, T, H, E, offset):
+    say("router bf16 operands", T, H, E, offset)
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T * H + offset, generator=g).to(torch.bfloat16).to(cuda)[offset:].view(T, H)
+    w = (0.05 * torch.randn(E, H, generator=g)).to(torch.bfloat16).to(cuda)
+    aff, lg = M.router(x, w.t(), 2, return_logits=True)
+    assert aff.dtype == lg.dtype == torch.float32
+    x64, w64 = np_f32(x).astype(np.float64), np_f32(w).astype(np.float64)
+    ref, scale = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
+    assert np.all(np.abs(np_f32(lg) - ref) <= 1e-6 * scale + 1e-6)
+    ids, wts = R.route_topk_act(np_f32(lg), 2, R.SOFTMAX)
+    assert np.array_equal(np_f32(aff), R.scatter_dense(ids, wts, E))
+
+
 def test_router_bf16_computation(cuda):
     say("router bf16 computation dtype")
     g = torch.Generator().manual_seed(4)

@@ -103,7 +103,12 @@ def router_logits(hidden_states, router_weights, router_bias=None, gamma=None, e
     hidden_states [T, H]; router_weights [H, E] as the reference passes them
     (used without a copy when they are the transpose view of a contiguous
     [E, H] parameter)."""
-    x = hidden_states.to(computation_dtype)
+    # bf16 operands of the fp32 linear step: a bf16 x bf16 product is exact in fp32 and both
+    # kernels sum in fp32, so the bf16 matrix cores serve, without a cast of x. Against 64 bits
+    # at 1500 tokens of 5120 and 160 experts 1.3e-7 (fp32 matrix cores 1.5e-7), in 19 against 50 us.
+    exact_bf16 = (computation_dtype == torch.float32 and gamma is None
+                  and hidden_states.dtype == torch.bfloat16 and router_weights.dtype == torch.bfloat16)
+    x = hidden_states if exact_bf16 else hidden_states.to(computation_dtype)
     if gamma is not None:
         if x.dtype == torch.float16:
             # fp32 norm, then the fp16 rounding _torch_rms_norm's cast back applies
@@ -115,7 +120,10 @@ def router_logits(hidden_states, router_weights, router_bias=None, gamma=None, e
         wt = wt.contiguous()
     bias = None if router_bias is None else router_bias.to(computation_dtype).float().contiguous()
     if x.dtype == torch.bfloat16 and wt.dtype == torch.bfloat16:
-        logits = ops.router_logits(x.contiguous(), wt, bias)
+        x = x.contiguous()
+        if exact_bf16 and x.data_ptr() % 16:
+            x = x.clone()  # the kernel reads 16 bytes at a time
+        logits = ops.router_logits(x, wt, bias)
     else:
         if computation_dtype != torch.float32 and wt.dtype != computation_dtype:
             # F.linear's operands are router_weights.to(computation_dtype) (router.py:419-424)
