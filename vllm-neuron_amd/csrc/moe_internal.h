@@ -42,7 +42,9 @@ constexpr int kMidTileRows = 64;
 constexpr int kMidTallRows = 128;
 constexpr int kMidMaxRows = 40;
 constexpr int kMidTallMaxRows = 76;
-// Work items (two per CU) from which they run 16-row tiles and small layers.
+// Work items from which they run 16-row tiles (four per CU), and 32-row tiles and small layers
+// (two per CU).
+constexpr long kMidMinItems16 = 1024;
 constexpr long kMidMinItems = 512;
 
 // Compute units of the current device (cached per device; 256 on MI355X), for
