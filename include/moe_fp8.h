@@ -368,6 +368,15 @@ int moe_expert_down_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, int I
                        const int32_t* num_tiles, int max_tiles, int mt, void* y_bf16,
                        void* stream);
 
+/* Which of the MXFP4 products run the block kernels on a list of at most max_tiles row tiles of
+ * mt rows, with 16-byte aligned operands and no shared experts: bit 0 gate_up, bit 1 down; the
+ * ring kernels run the others. Host only. */
+int moe_mx_row_tile_kernels(int H, int I, int E, int max_tiles, int mt);
+
+/* Rows per tile of the MXFP4 layer's expert tiles: 16, 32 or 64 (row tiles), or 128 (block
+ * tiles, which always run the block kernels). Host only. */
+int moe_layer_mx_tile_rows(int T, int H, int I, int E, int K, int B);
+
 /* The MoE layer with MX experts (GPT-OSS: MXFP4 experts with biases, Swish and
  * clamps): [residual add ->] [RMSNorm (gamma) ->] router logits (+ router_bias) ->
  * top-k (orders TOPK_ACT / ACT_TOPK) -> mapping -> MXFP8 activations -> MX gate_up

@@ -1,0 +1,36 @@
+"""Which kernels the MXFP4 experts run, by sizes: host rules, no GPU needed. The results of both
+kernels are the same bits (test_gpu_mx_block.py); these are the sizes where one of them was
+measured slower."""
+import pytest
+
+from vllm_neuron_amd import _lib
+
+RING, GATE_UP, DOWN, BOTH = 0, 1, 2, 3
+
+
+def _plan(T, H, I, E, K, B=256):
+    """(rows per tile, products on the block kernels) of the layer on row tiles."""
+    lib = _lib.load()
+    mt = lib.moe_layer_mx_tile_rows(T, H, I, E, K, B)
+    tiles = lib.moe_max_tiles(T, K, E, lib.moe_num_blocks(T, K, E, B), B, 0, mt)
+    return mt, lib.moe_mx_row_tile_kernels(H, I, E, tiles, mt)
+
+
+# GPT-OSS-20B (32 experts, top-4, 2880 padded to 3072): one tile per expert is 768 gate_up and 384
+# down items. Three whole rounds of the ring kernels' 256 workgroups, and 64-row tiles whose down
+# would stay on the ring.
+@pytest.mark.parametrize("T,rows,on_block", [
+    (32, 16, RING), (33, 32, RING), (64, 32, RING), (80, 32, DOWN), (135, 32, DOWN), (160, 64, BOTH),
+    (256, 64, BOTH)])
+def test_gpt_oss_20b_row_tiles(T, rows, on_block):
+    assert _plan(T, 3072, 3072, 32, 4) == (rows, on_block)
+
+
+@pytest.mark.parametrize("T,H,I,E,rows,on_block", [
+    (48, 4096, 4096, 24, 32, RING),        # 768 gate_up items of K = 4096
+    (108, 1024, 1024, 96, 32, GATE_UP),    # of K = 1024: the block kernel even at 768; down on the ring
+    (144, 1024, 512, 128, 64, BOTH),       # 512 and 512: one round of the block kernels
+    (320, 1024, 2048, 64, 64, GATE_UP),    # 20 rows per expert: 64-row tiles, down on the ring
+    (160, 3072, 3072, 128, 64, BOTH)])     # GPT-OSS-120B
+def test_row_tiles(T, H, I, E, rows, on_block):
+    assert _plan(T, H, I, E, 4) == (rows, on_block)

@@ -406,6 +406,36 @@ extern "C" int moe_layer_forward_noalloc(
                             logits_out, ws, (size_t)MOE_NOALLOC_SCRATCH_BYTES, stream);
 }
 
+// Rows per tile of the MX layer's row tiles; block_ok: the block kernels fit its products.
+static int mx_layer_rows(int T, int H, int I, int E, int K, int B, bool block_ok) {
+  const int mt = choose_mt_mx(T, K, E), N = moe_num_blocks(T, K, E, B);
+  if (!block_ok || mt != 32) return mt;
+  // Of 5 to 24 rows per expert, 64-row tiles keep nearly every expert in one tile: where the block
+  // kernels run both products on them, and from 9 rows where they run gate_up on them and down
+  // on neither height (64 experts of 1024 x 2048, 20 rows: 87 -> 75 us). With down on the ring
+  // kernels they lose below that (160 experts of 512 x 1024, 5 / 8 rows: 57.2 / 65.5 at 32 rows, 62.9 /
+  // 69.7 us at 64), and where the ring keeps gate_up at 32 rows (GPT-OSS-20B, 33 / 64 / 80 / 135
+  // tokens 117 / 120 / 114 / 118 at 32 rows, 125 / 127 / 128 / 130 us at 64).
+  const int t32 = moe_max_tiles(T, K, E, N, B, 0, 32), t64 = moe_max_tiles(T, K, E, N, B, 0, 64);
+  auto on_block = [&](int kind, int rows) {
+    return mx_rows_on_block(kind, H, I, E, rows == 32 ? t32 : t64, rows);
+  };
+  if (!on_block(0, 32) || !on_block(0, 64)) return 32;
+  const bool tall = on_block(1, 64) || (!on_block(1, 32) && routed_rows(T, K, E) > 8L * E);
+  return tall ? 64 : 32;
+}
+
+extern "C" int moe_layer_mx_tile_rows(int T, int H, int I, int E, int K, int B) {
+  if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || K <= 0 || B <= 0) return 0;
+  MxArgs a{};
+  a.T = T;
+  a.H = H;
+  a.I = I;
+  a.rows = routed_rows(T, K, E);
+  const bool block_ok = mx_block_fits(0, a) && mx_block_fits(1, a);
+  return use_block(T, K, E) && block_ok ? kMxBlockTileRows : mx_layer_rows(T, H, I, E, K, B, block_ok);
+}
+
 // ---------------------------------------------------------------------------
 // The layer with MX experts (GPT-OSS): [residual add ->] [RMSNorm ->] router ->
 // top-k -> mapping (compact rows) -> MXFP8 quantization -> MX gate_up (bias,
@@ -478,9 +508,7 @@ extern "C" int moe_layer_forward_mx(
   bd.y = w.y;
   const bool block_ok = wfmt == MOE_MX_FP4 && (act == MOE_ACT_SILU || act == MOE_ACT_SWISH) &&
                         mx_block_fits(0, bg) && mx_block_fits(1, bd);
-  int mt = choose_mt_mx(T, K, E);
-  // where the block kernels run both heights, 64 rows keep nearly every expert in one tile
-  if (block_ok && mt == 32 && (long)moe_max_tiles(T, K, E, N, B, 0, 64) * (I / 128) >= kMidMinItems) mt = 64;
+  const int mt = mx_layer_rows(T, H, I, E, K, B, block_ok);
   const int max_tiles = moe_max_tiles(T, K, E, N, B, 0, mt);
   float* logits = logits_out ? logits_out : w.logits;
   int32_t* ids = ids_out ? ids_out : w.ids;

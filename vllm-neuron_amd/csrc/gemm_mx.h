@@ -45,7 +45,21 @@ struct MxArgs {
 // of 512, no shared experts, 16-byte aligned operands that 32-bit byte offsets reach).
 bool mx_block_fits(int kind, const MxArgs& a);
 void launch_mx_block(int kind, const MxArgs& a, int max_tiles, hipStream_t st);
-
+// Whether the MXFP4 product `kind` runs the block kernels on a list of max_tiles row tiles of mt
+// rows, where mx_block_fits; otherwise the ring kernels. They run from two items per CU on, but for
+// 32-row tiles of long K where three whole rounds of the ring's one workgroup per CU hold one tile
+// per expert: there the block kernels' two workgroups per CU are one and a half rounds. Alone, us,
+// ring -> block, 8 rows per expert: gate_up K = 3072, 512 / 640 / 704 / 768 / 800 items 44.2 / 62.5 /
+// 63.5 / 64.5 / 80.9 -> 37.1 / 58.9 / 61.7 / 64.1 / 64.9; down K = 3072, 512 / 576 / 640 / 768 / 800
+// items 43.4 / 57.4 / 58.3 / 61.0 / 75.8 -> 38.0 / 56.8 / 59.8 / 64.9 / 66.1; K = 1024, 768 items 27.6
+// -> 23.9 and 22.8 -> 22.8. gate_up loses in whole layers (32 experts of K = 3072, 24 of K = 4096).
+inline bool mx_rows_on_block(int kind, int H, int I, int E, int max_tiles, int mt) {
+  const long cols = (kind == 0) ? I / 128 : H / 256;
+  if ((mt != 32 && mt != 64) || max_tiles * cols < kMidMinItems) return false;
+  const bool one_each = 5L * max_tiles <= 8L * E;  // up to 19 of 32 rows on average
+  return !(mt == 32 && (kind == 0 ? H : I) > 2048 && one_each && E * cols > (kind == 0 ? 704 : 576) &&
+           E * cols <= 768);
+}
 
 __device__ __forceinline__ v4f mfma_mx(const v8i& a, const v8i& b, const v4f& c, int sa, int sb,
                                       std::integral_constant<int, kFmtFp8>) {

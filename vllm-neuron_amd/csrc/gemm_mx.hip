@@ -835,12 +835,11 @@ __global__ __launch_bounds__(64 * kDownCombineMaxK) void down_combine_mx_one_ker
 
 template <int KIND, int WFMT>
 static int launch_mx(const MxArgs& a, int max_tiles, int mt, hipStream_t st) {
-  // MXFP4 tiles of 32 and 64 rows, enough of them to fill the chip twice: the block kernels
-  // (two workgroups per CU, the same output bits). GPT-OSS-120B layer, ring -> block kernels:
+  // MXFP4 tiles of 32 and 64 rows, enough of them to fill the chip twice (mx_rows_on_block): the
+  // block kernels (two workgroups per CU, the same output bits). GPT-OSS-120B layer, ring -> block kernels:
   // 160 tokens 380 -> 329 us, 512 424 -> 361 us, 1000 534 -> 402 us; at 16-row tiles the ring
   // is the faster (128 tokens 316 against 325 us, 48 tokens 270 against 281 us).
-  if (WFMT == kFmtFp4 && (mt == 32 || mt == 64) &&
-      (long)max_tiles * ((KIND == 0) ? a.I / 128 : a.H / 256) >= kMidMinItems) {
+  if (WFMT == kFmtFp4 && mx_rows_on_block(KIND, a.H, a.I, a.E, max_tiles, mt)) {
     MxArgs b = a;
     b.rows = a.NB;
     if (mx_block_fits(KIND, b)) {
@@ -924,6 +923,17 @@ static int mx_common_checks(const char* _moe_fn, int T, int H, int I, int E, int
   MOE_CHECK_SUPPORTED(mt != 128, "MX expert tiles stop at 64 rows (mt=128 is not built)");
   MOE_CHECK_ARG(wfmt == MOE_MX_FP4 || wfmt == MOE_MX_FP8, "weight format must be MOE_MX_FP4 or MOE_MX_FP8");
   return MOE_OK;
+}
+
+extern "C" int moe_mx_row_tile_kernels(int H, int I, int E, int max_tiles, int mt) {
+  if (H <= 0 || I <= 0 || E <= 0 || max_tiles <= 0) return 0;
+  MxArgs a{};
+  a.H = H;
+  a.I = I;
+  int on_block = 0;
+  for (int kind = 0; kind < 2; ++kind)
+    on_block |= (mx_rows_on_block(kind, H, I, E, max_tiles, mt) && mx_block_fits(kind, a)) << kind;
+  return on_block;
 }
 
 static inline float lim(float v, float dflt) { return isnan(v) ? dflt : v; }
