@@ -11,7 +11,7 @@ import torch
 
 from _util import say
 from test_gpu_mx import make_mx_weights
-from vllm_neuron_amd import ops
+from vllm_neuron_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +53,30 @@ def test_layer_equals_ring_kernels(cuda, T, E, K, H, I, act, bias, skew):
     gl, ul = ((None, 7.0), (-6.0, 8.0)) if act == "swish" else ((None, None), (None, None))
     assert T * K > 32 * E
     out, ids, wts, _ = ops.layer_forward_mx(x, w, K, act, gl, ul, return_routing=True)
+    ref = _ring_experts(x, ids, wts, w, act, gl, ul)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    assert bool(torch.isfinite(out.float()).all()) and float(out.float().abs().max()) > 0
+
+
+# Enough items for block tiles: experts of every count of 16-row fragments, of two and three tiles,
+# and of none (each token names its expert in the first E columns).
+@pytest.mark.parametrize("H,I,act,bias", [(512, 1536, "swish", True), (1024, 1024, "silu", False),
+                                          (1536, 2048, "swish", True)])
+def test_layer_block_tiles_of_every_height(cuda, H, I, act, bias):
+    counts = [1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 127, 128, 0, 129, 256, 257]
+    E, T = len(counts), sum(counts)
+    say("mx block tiles", H, I, act, T)
+    assert _lib.load().moe_layer_mx_tile_rows(T, H, I, E, 1, 256) == 128
+    w = make_mx_weights(E, H, I, 19, cuda, bias=bias)
+    w = dataclasses.replace(w, router_w=torch.eye(E, H, dtype=torch.bfloat16, device=cuda), router_bias=None)
+    g = torch.Generator().manual_seed(T)
+    e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)]
+    x = torch.randn(T, H, generator=g)
+    x[:, :E] = 8.0 * torch.nn.functional.one_hot(e, E)
+    x = x.to(torch.bfloat16).to(cuda)
+    gl, ul = ((None, 7.0), (-6.0, 8.0)) if act == "swish" else ((None, None), (None, None))
+    out, ids, wts, _ = ops.layer_forward_mx(x, w, 1, act, gl, ul, return_routing=True)
+    assert torch.equal(ids.flatten().cpu().long(), e)
     ref = _ring_experts(x, ids, wts, w, act, gl, ul)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     assert bool(torch.isfinite(out.float()).all()) and float(out.float().abs().max()) > 0

@@ -425,6 +425,21 @@ static int mx_layer_rows(int T, int H, int I, int E, int K, int B, bool block_ok
   return tall ? 64 : 32;
 }
 
+// Whether the MXFP4 layer runs block tiles: above 32 rows per expert, up to 40 of them (an expert is
+// one tile of the ring kernels too), or where 64-row tiles are more than one round of the ring
+// kernels' one workgroup per CU in one product (from 320 items, counted with a remainder tile for
+// each expert). In one round a taller tile is only a longer chain. Layer, 64-row
+// tiles on the ring -> block tiles, us: 4 experts of 512 x 512 at 33 / 50 / 64 / 100 / 256 rows per
+// expert 35.8 / 36.3 / 36.9 / 37.2 / 43.3 -> 32.2 / 34.0 / 36.7 / 41.1 / 47.2; 8 of 1024 x 1024 at 40 / 80 /
+// 200 / 256 (264 and 320 items) 43.3 / 50.6 / 54.0 / 65.7 -> 40.8 / 53.3 / 54.3 / 56.9; 4 of 3072 x 3072
+// at 128 / 150 (288 and 336 items) 71.3 / 98.7 -> 80.2 / 74.5.
+constexpr long kMxBlockMinItems = 320;
+static bool mx_layer_block(int T, int H, int I, int E, int K, int B) {
+  if (!use_block(T, K, E)) return false;
+  const long R = routed_rows(T, K, E), tiles = (R + std::min(64, B) - 1) / std::min(64, B) + E;
+  return R <= 40L * E || tiles * std::max(I / 128, H / 256) >= kMxBlockMinItems;
+}
+
 extern "C" int moe_layer_mx_tile_rows(int T, int H, int I, int E, int K, int B) {
   if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || K <= 0 || B <= 0) return 0;
   MxArgs a{};
@@ -433,7 +448,8 @@ extern "C" int moe_layer_mx_tile_rows(int T, int H, int I, int E, int K, int B) 
   a.I = I;
   a.rows = routed_rows(T, K, E);
   const bool block_ok = mx_block_fits(0, a) && mx_block_fits(1, a);
-  return use_block(T, K, E) && block_ok ? kMxBlockTileRows : mx_layer_rows(T, H, I, E, K, B, block_ok);
+  return block_ok && mx_layer_block(T, H, I, E, K, B) ? kMxBlockTileRows
+                                                      : mx_layer_rows(T, H, I, E, K, B, block_ok);
 }
 
 // ---------------------------------------------------------------------------
@@ -525,11 +541,10 @@ extern "C" int moe_layer_forward_mx(
     moe::set_error(_moe_fn, "%s", saved);                      \
     return rc;                                                 \
   }
-  // Above 32 rows per expert the MXFP4 experts run the block kernels: their tiles go
-  // into the row-tile list's room (at most R / 128 + E of them, which is no more than the
-  // R / 64 + N row tiles it is sized for, N >= E), their segments (8 bytes each) into the
-  // fp8 block tiles' (24 bytes for each of NB / 256 + E, NB >= R).
-  const bool block = use_block(T, K, E) && block_ok;
+  // Block tiles go into the row-tile list's room (at most R / 128 + E of them, which is no more
+  // than the R / 64 + N row tiles it is sized for, N >= E), their segments (8 bytes each) into
+  // the fp8 block tiles' (24 bytes for each of NB / 256 + E, NB >= R).
+  const bool block = block_ok && mx_layer_block(T, H, I, E, K, B);
   const int mbt = block ? mx_block_max_tiles(T, K, E) : 0;
   TileOut to{};
   to.tiles = (int4*)w.tiles;
