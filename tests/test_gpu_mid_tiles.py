@@ -22,11 +22,13 @@ def _experts(tpid, b2e, B, T, K, E, S, mt, xq, xs, w):
 
 # Expert counts that give every tile height around a 16-row fragment and a 64-row tile; mt 128
 # runs the ring kernel. H and I: one group of four K blocks, several, and odd numbers of them.
-# At mt 32 the last case has the 512 items from which these kernels take it, the first has not.
-@pytest.mark.parametrize("H,I,S,chan", [(512, 512, 0, False), (1024, 1536, 1, False), (1536, 512, 2, True),
-                                        (512, 8192, 1, False)])
+# 64-row tiles always take these kernels, 32-row tiles from 512 items of a product (mid32: bit 0
+# gate_up, bit 1 down).
+@pytest.mark.parametrize("H,I,S,chan,mid32", [(512, 512, 0, False, 0), (1024, 1536, 1, False, 1),
+                                              (1536, 512, 2, True, 0), (512, 8192, 1, False, 1),
+                                              (4096, 512, 1, False, 2), (4096, 1536, 1, True, 3)])
 @pytest.mark.parametrize("mt", [32, 64])
-def test_row_tiles_equal_ring_kernel(cuda, mt, H, I, S, chan):
+def test_row_tiles_equal_ring_kernel(cuda, mt, H, I, S, chan, mid32):
     counts = [1, 15, 16, 17, 0, 31, 32, 33, 48, 49, 63, 64, 65, 130]
     E, T = len(counts), sum(counts)
     say("mid row tiles", mt, H, I, S, chan, T)
@@ -41,6 +43,8 @@ def test_row_tiles_equal_ring_kernel(cuda, mt, H, I, S, chan):
     m = ops.blockwise_mapping(ids=ids, n_experts=E, block_size=256)
     tpid, b2e = m["token_position_to_id"].clone(), m["block_to_expert"]
     tpid[(tpid >= 0).nonzero()[5]] = -1  # a hole inside a tile: its h row is not written
+    tiles = ops.build_tiles(tpid, b2e, 256, T, 1, E, S, 32)[2]
+    assert (tiles * (I // 128) >= 512) + 2 * (tiles * (H // 256) >= 512) == mid32
     xq, xs = ops.act_quant(synthetic.hidden_states(T, H, 3).to(cuda))
     got = _experts(tpid, b2e, 256, T, 1, E, S, mt, xq, xs, w)
     ref = _experts(tpid, b2e, 256, T, 1, E, S, 128, xq, xs, w)

@@ -1,5 +1,5 @@
-"""The MXFP4 block kernels: of the layer above 32 routed rows per expert (block tiles), and of
-32- and 64-row tiles of at least 512 work items.
+"""The MXFP4 block kernels: of the layer's block tiles (above 32 routed rows per expert, enough
+items), and of 32- and 64-row tiles of at least 512 work items.
 
 Same scaled MFMAs in the same K order and the same epilogue arithmetic as the ring kernels,
 so results are held bit for bit to those on 16-row tiles, which always run them (and which
@@ -35,7 +35,8 @@ def _ring_experts(x, ids, wts, w, act, gl, ul, B=256):
 
 
 # T * K / E > 32 in all of them. H = I = 512: one scale group, two steps; 1536 x 1024: odd
-# numbers of groups; 768: not a multiple of 512, which stays on the row-tile kernels.
+# numbers of groups; 768: not a multiple of 512, which stays on the row-tile kernels. The first
+# and 1025 tokens run block tiles, the others have too few items for them.
 @pytest.mark.parametrize("T,E,K,H,I,act,bias,skew", [
     (67, 2, 1, 512, 512, "swish", True, [0.0, -60.0]),         # one expert holds all 67 rows, one none
     (129, 4, 2, 512, 512, "silu", False, [30.0, 0.0, 0.0, -30.0]),  # a 129-row expert: two 65-row tiles
@@ -83,20 +84,31 @@ def test_layer_block_tiles_of_every_height(cuda, H, I, act, bias):
 
 
 # 5 to 32 rows per expert: row tiles (the layer's, and the operator path's at 32 or 64 rows).
-@pytest.mark.parametrize("T,E,K,H,I,act,B", [
-    (160, 128, 4, 512, 512, "swish", 256),
-    (700, 160, 4, 512, 1024, "silu", 256),
-    (900, 128, 4, 1024, 512, "swish", 16),   # 16-slot blocks: every tile at most 16 rows
-    (200, 40, 4, 512, 512, "swish", 256),    # too few items: the ring kernels
+# on_block: the products on the block kernels, bit 0 gate_up, bit 1 down (the same for both lists).
+@pytest.mark.parametrize("T,E,K,H,I,act,B,rows,on_block", [
+    (160, 128, 4, 512, 512, "swish", 256, 32, 1),
+    (700, 160, 4, 512, 1024, "silu", 256, 32, 3),
+    (300, 136, 4, 1024, 1024, "silu", 256, 64, 3),   # the operator path: 32 rows
+    (1200, 160, 4, 1024, 512, "swish", 256, 64, 3),  # 30 rows per expert: 64 rows in both
+    (250, 64, 4, 2560, 1536, "swish", 256, 32, 2),
+    (900, 128, 4, 1024, 512, "swish", 16, 64, 3),   # 16-slot blocks: every tile at most 16 rows
+    (200, 40, 4, 512, 512, "swish", 256, 32, 0),    # too few items: the ring kernels
 ])
-def test_row_tiles_equal_ring_kernels(cuda, T, E, K, H, I, act, B):
+def test_row_tiles_equal_ring_kernels(cuda, T, E, K, H, I, act, B, rows, on_block):
     say("mx block row tiles", T, E, K, H, I, act, B)
+    lib = _lib.load()
+    assert lib.moe_layer_mx_tile_rows(T, H, I, E, K, B) == rows
+    for mt in (rows, ops.choose_mt(T, K, E)):
+        tiles = lib.moe_max_tiles(T, K, E, lib.moe_num_blocks(T, K, E, B), B, 0, mt)
+        assert lib.moe_mx_row_tile_kernels(H, I, E, tiles, mt) == on_block
     w = make_mx_weights(E, H, I, 13, cuda)
     g = torch.Generator().manual_seed(T)
     x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(cuda)
     gl, ul = ((None, 7.0), (-6.0, 8.0)) if act == "swish" else ((None, None), (None, None))
     assert 4 * E < T * K <= 32 * E
     out, ids, wts, _ = ops.layer_forward_mx(x, w, K, act, gl, ul, return_routing=True, block_size=B)
+    heights = torch.bincount(ids.flatten(), minlength=E).clamp(max=rows)
+    assert B < 64 or int(heights.max()) > 16
     ref = _ring_experts(x, ids, wts, w, act, gl, ul, B)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     got = ops.mx_experts(x, ids, wts, w, act, gl, ul, block_size=B)
