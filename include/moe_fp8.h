@@ -368,6 +368,11 @@ int moe_expert_down_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, int I
                        const int32_t* num_tiles, int max_tiles, int mt, void* y_bf16,
                        void* stream);
 
+/* Rows per tile of the fp8 layer's expert tiles: 16, 32 or 64 (row tiles, up to 32 routed rows
+ * per expert), above that 64 or 128 (block tiles of the mid-size kernels) or 256 (of the block
+ * kernels). Host only. */
+int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B);
+
 /* Which of the MXFP4 products run the block kernels on a list of at most max_tiles row tiles of
  * mt rows, with 16-byte aligned operands and no shared experts: bit 0 gate_up, bit 1 down; the
  * ring kernels run the others. Host only. */

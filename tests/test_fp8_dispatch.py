@@ -1,0 +1,22 @@
+"""Rows per tile of the fp8 layer, by sizes: host rules, no GPU needed. The results of all tile
+heights are the same bits (test_gpu_mid_tiles.py); these are the sizes where one of them was
+measured slower."""
+import pytest
+
+from vllm_neuron_amd import _lib
+
+
+def _rows(T, H, I, E, K, S=0, B=256):
+    return _lib.load().moe_layer_tile_rows(T, H, I, E, K, S, B)
+
+
+# 5 to 24 rows per expert: 64-row tiles only where both products have 512 items of them.
+@pytest.mark.parametrize("T,H,I,E,K,S,rows", [
+    (16, 4096, 14336, 8, 2, 0, 16), (24, 4096, 14336, 8, 2, 0, 32),  # 1008 gate_up, 144 down items
+    (96, 4096, 14336, 8, 2, 0, 32), (112, 4096, 14336, 8, 2, 0, 64),
+    (96, 7168, 2048, 32, 8, 1, 64),   # 47 tiles: 752 and 1316
+    (257, 7168, 2048, 256, 8, 1, 64), (200, 5120, 1536, 160, 8, 1, 64),
+    (20, 1024, 512, 8, 2, 0, 32), (100, 1024, 512, 8, 2, 0, 64),  # the small layer
+    (200, 2048, 768, 128, 8, 0, 32)])  # I not a multiple of 512
+def test_row_tiles(T, H, I, E, K, S, rows):
+    assert _rows(T, H, I, E, K, S) == rows

@@ -157,6 +157,40 @@ static RouterFuse map_fuse(const LayerWs& w, int B, int N, const TileOut& to) {
   return fz;
 }
 
+// Rows per tile of the fp8 layer's row tiles; mid_ok: the mid-size kernels fit its products.
+static int layer_rows(int T, int H, int I, int E, int K, int n_shared, int B, bool mid_ok) {
+  const int mt = choose_mt(T, K, E);
+  if (!mid_ok || mt != 32) return mt;
+  // Of 5 to 24 rows per expert, 64-row tiles keep nearly every expert in one tile, where both
+  // products then have enough items. With few items of down, its 32-row tiles stay on the ring
+  // kernels: 8 experts of 4096 x 14336 (128 down items of K = 14336), 24 / 48 / 96 tokens, gate_up and
+  // down on the ring 293 / 296 / 305, both on 64-row tiles 343 / 345 / 350, so 268 / 270 / 276 us.
+  const int t64 = moe_max_tiles(T, K, E, moe_num_blocks(T, K, E, B), B, n_shared, kMidTileRows);
+  return (long)t64 * std::min(I / 128, H / 256) >= kMidMinItems ? kMidTileRows : mt;
+}
+
+// Rows per tile of the fp8 layer's block tiles on the mid-size kernels, where they fit; 0: the
+// layer runs the 256-row block kernels or row tiles.
+static int layer_mid_rows(int T, int I, int E, int K, int n_shared) {
+  const long R = routed_rows(T, K, E);
+  if (!use_block(T, K, E) || R > kMidTallMaxRows * (long)E) return 0;
+  const int rows = R <= kMidMaxRows * (long)E ? kMidTileRows : kMidTallRows;
+  return (long)mid_max_tiles(T, K, E, n_shared, rows) * (I / 128) >= kMidMinItems ? rows : 0;
+}
+
+extern "C" int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B) {
+  if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || K <= 0 || n_shared < 0 || B <= 0) return 0;
+  MidArgs a{};
+  a.T = T;
+  a.H = H;
+  a.I = I;
+  a.rows = routed_rows(T, K, E) + (long)n_shared * T;
+  const bool mid_ok = mid_fits(0, a) && mid_fits(1, a);
+  if (!use_block(T, K, E)) return layer_rows(T, H, I, E, K, n_shared, B, mid_ok);
+  const int rows = mid_ok ? layer_mid_rows(T, I, E, K, n_shared) : 0;
+  return rows ? rows : kBlockTileRows;
+}
+
 // The layer forward of both entry points: `workspace` is the caller's buffer or
 // this device's static scratch. _moe_fn names the entry point in error messages.
 static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const void* residual_bf16,
@@ -220,11 +254,7 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   md.wssh = w2_shared_scale;
   md.y = w.y;
   const bool mid_ok = mid_fits(0, mg) && mid_fits(1, md);
-  int mt = choose_mt(T, K, E);
-  // where the mid-size kernels run both heights, 64 rows keep nearly every expert in one tile
-  if (mid_ok && mt == 32 &&
-      (long)moe_max_tiles(T, K, E, N, B, n_shared, kMidTileRows) * (I / 128) >= kMidMinItems)
-    mt = kMidTileRows;
+  const int mt = layer_rows(T, H, I, E, K, n_shared, B, mid_ok);
   const int max_tiles = moe_max_tiles(T, K, E, N, B, n_shared, mt);
   float* logits = logits_out ? logits_out : w.logits;
   int32_t* ids = ids_out ? ids_out : w.ids;
@@ -245,10 +275,10 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   // Above 32 and up to kMidTallMaxRows rows per expert on average, 64- or 128-row block
   // tiles: their list goes into the row-tile list's room (sized for 64-row tiles), its segments
   // (8 bytes each) into the block tiles' (24 bytes each).
-  const int mid_rows = R <= kMidMaxRows * (long)E ? kMidTileRows : kMidTallRows;
-  const int mmt = block ? mid_max_tiles(T, K, E, n_shared, mid_rows) : 0;
-  const bool mid = block && R <= kMidTallMaxRows * (long)E && mid_ok && (long)mmt * (I / 128) >= kMidMinItems &&
-                   mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) && mmt <= 3L * mbt;
+  const int mid_rows = mid_ok ? layer_mid_rows(T, I, E, K, n_shared) : 0;
+  const int mmt = mid_rows ? mid_max_tiles(T, K, E, n_shared, mid_rows) : 0;
+  const bool mid = mid_rows != 0 && mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) &&
+                   mmt <= 3L * mbt;
   TileOut to{};
   if (mid) {
     to.tiles = (int4*)w.tiles;
