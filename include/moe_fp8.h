@@ -369,7 +369,7 @@ int moe_expert_down_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, int I
                        void* stream);
 
 /* Rows per tile of the fp8 layer's expert tiles: 16, 32 or 64 (row tiles, up to 32 routed rows
- * per expert), above that 64 or 128 (block tiles of the mid-size kernels) or 256 (of the block
+ * per expert), above that 128 (block tiles of the mid-size kernels) or 256 (of the block
  * kernels). Host only. */
 int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B);
 

@@ -20,3 +20,13 @@ def _rows(T, H, I, E, K, S=0, B=256):
     (200, 2048, 768, 128, 8, 0, 32)])  # I not a multiple of 512
 def test_row_tiles(T, H, I, E, K, S, rows):
     assert _rows(T, H, I, E, K, S) == rows
+
+
+# Above 32: 128-row block tiles up to 76 rows per expert, where their gate_up items fill the chip twice.
+@pytest.mark.parametrize("T,H,I,E,K,S,rows", [
+    (1537, 7168, 2048, 384, 8, 1, 128), (1901, 7168, 2048, 384, 8, 1, 128), (3648, 7168, 2048, 384, 8, 1, 128),
+    (3649, 7168, 2048, 384, 8, 1, 256), (641, 5120, 1536, 160, 8, 1, 128), (8192, 7168, 2048, 256, 8, 1, 256),
+    (136, 7168, 2048, 32, 8, 1, 128),                                   # 41 x 16 items
+    (160, 1024, 512, 8, 2, 0, 256), (520, 2048, 768, 128, 8, 0, 256)])  # 10 x 4; I not a multiple of 512
+def test_block_tiles(T, H, I, E, K, S, rows):
+    assert _rows(T, H, I, E, K, S) == rows

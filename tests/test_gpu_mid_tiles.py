@@ -75,8 +75,8 @@ def test_sixteen_row_tiles_equal_ring_kernel(cuda):
 
 
 # 33 to 76 rows per expert: the layer against the op-by-op path's block kernels. A zero weight
-# scale repeats the previous block's ratio in both. Above 40 rows (128-row tiles) a router
-# bias spreads the experts over every count of 16-row fragments and several tiles.
+# scale repeats the previous block's ratio in both. Above 40 rows a router bias spreads the
+# experts over every count of 16-row fragments and several tiles.
 @pytest.mark.parametrize("T,S,zero", [(513, 1, False), (577, 0, True), (640, 1, True), (641, 1, False),
                                       (1000, 0, True), (1216, 2, False)])
 def test_layer_block_tiles_equal_block_kernels(cuda, T, S, zero):

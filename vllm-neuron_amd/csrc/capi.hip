@@ -169,13 +169,10 @@ static int layer_rows(int T, int H, int I, int E, int K, int n_shared, int B, bo
   return (long)t64 * std::min(I / 128, H / 256) >= kMidMinItems ? kMidTileRows : mt;
 }
 
-// Rows per tile of the fp8 layer's block tiles on the mid-size kernels, where they fit; 0: the
-// layer runs the 256-row block kernels or row tiles.
-static int layer_mid_rows(int T, int I, int E, int K, int n_shared) {
-  const long R = routed_rows(T, K, E);
-  if (!use_block(T, K, E) || R > kMidTallMaxRows * (long)E) return 0;
-  const int rows = R <= kMidMaxRows * (long)E ? kMidTileRows : kMidTallRows;
-  return (long)mid_max_tiles(T, K, E, n_shared, rows) * (I / 128) >= kMidMinItems ? rows : 0;
+// Whether the fp8 layer runs the mid-size kernels on block tiles, where they fit.
+static bool layer_mid(int T, int I, int E, int K, int n_shared) {
+  return use_block(T, K, E) && routed_rows(T, K, E) <= kMidTallMaxRows * (long)E &&
+         (long)mid_max_tiles(T, K, E, n_shared) * (I / 128) >= kMidMinItems;
 }
 
 extern "C" int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B) {
@@ -187,8 +184,7 @@ extern "C" int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shar
   a.rows = routed_rows(T, K, E) + (long)n_shared * T;
   const bool mid_ok = mid_fits(0, a) && mid_fits(1, a);
   if (!use_block(T, K, E)) return layer_rows(T, H, I, E, K, n_shared, B, mid_ok);
-  const int rows = mid_ok ? layer_mid_rows(T, I, E, K, n_shared) : 0;
-  return rows ? rows : kBlockTileRows;
+  return mid_ok && layer_mid(T, I, E, K, n_shared) ? kMidTallRows : kBlockTileRows;
 }
 
 // The layer forward of both entry points: `workspace` is the caller's buffer or
@@ -272,20 +268,19 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   // The mapping also writes the expert tile list, from the counts.
   const bool block = use_block(T, K, E);
   const int mbt = block ? moe_max_block_tiles(T, K, E, N, B, n_shared) : 0;
-  // Above 32 and up to kMidTallMaxRows rows per expert on average, 64- or 128-row block
-  // tiles: their list goes into the row-tile list's room (sized for 64-row tiles), its segments
-  // (8 bytes each) into the block tiles' (24 bytes each).
-  const int mid_rows = mid_ok ? layer_mid_rows(T, I, E, K, n_shared) : 0;
-  const int mmt = mid_rows ? mid_max_tiles(T, K, E, n_shared, mid_rows) : 0;
-  const bool mid = mid_rows != 0 && mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) &&
-                   mmt <= 3L * mbt;
+  // Above 32 and up to kMidTallMaxRows rows per expert on average, 128-row block tiles: their
+  // list goes into the row-tile list's room (sized for 64-row tiles), its segments (8 bytes each)
+  // into the block tiles' (24 bytes each).
+  const int mmt = block ? mid_max_tiles(T, K, E, n_shared) : 0;
+  const bool mid = mid_ok && layer_mid(T, I, E, K, n_shared) &&
+                   mmt <= moe_max_tiles(T, K, E, N, B, n_shared, choose_mt_mx(T, K, E)) && mmt <= 3L * mbt;
   TileOut to{};
   if (mid) {
     to.tiles = (int4*)w.tiles;
     to.seg = (int2*)w.btiles;
     to.num_tiles = w.bnum;
     to.max_tiles = mmt;
-    to.mt = mid_rows;
+    to.mt = kMidTallRows;
     to.span = 1;
   } else if (block) {
     to.tiles = (int4*)w.btiles;
@@ -327,8 +322,8 @@ static int layer_forward_impl(const char* _moe_fn, const void* x_bf16, const voi
   if (mid) {
     MOE_CHECK_ARG(n_shared == 0 || (w13_shared && w13_shared_scale && w2_shared && w2_shared_scale),
                   "shared weights missing");
-    launch_mid(0, mg, mmt, mid_rows, (hipStream_t)stream);
-    launch_mid(1, md, mmt, mid_rows, (hipStream_t)stream);
+    launch_mid(0, mg, mmt, (hipStream_t)stream);
+    launch_mid(1, md, mmt, (hipStream_t)stream);
   } else if (block) {
     MOE_STEP(moe_expert_gate_up_block(w.xq, w.xs, T, H, I, E, w13, w13_scale, nullptr, w13_shared,
                                       w13_shared_scale, nullptr, n_shared, w.tpid, (int)NB, w.btiles,

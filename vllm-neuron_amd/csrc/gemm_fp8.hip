@@ -488,7 +488,7 @@ static int launch_gemm(const GemmArgs& a, int max_tiles, int mt, hipStream_t st)
     m.NB = a.NB;
     m.rows = a.NB + (long)a.nsh * a.T;
     if (mid_fits(KIND, m)) {
-      launch_mid(KIND, m, max_tiles, kMidTileRows, st);
+      launch_mid(KIND, m, max_tiles, st);
       return MOE_OK;
     }
   }

@@ -887,7 +887,7 @@ static void launch_block_rows(const BlkArgs& a, int tile_rows, int max_tiles, hi
   m.NB = a.NB;
   m.rows = a.NB + (long)a.nsh * a.T;
   if (tile_rows == kMidTallRows && a.cs == nullptr && a.cssh == nullptr && mid_fits(KIND, m))
-    launch_mid(KIND, m, max_tiles, kMidTallRows, st);
+    launch_mid(KIND, m, max_tiles, st);
   else
     launch_block<KIND>(a, max_tiles, st);
 }

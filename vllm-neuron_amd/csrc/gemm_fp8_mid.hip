@@ -1,5 +1,5 @@
-// FP8-blockwise expert GEMMs on tiles of up to 64 or 128 rows, between one-token decode and
-// prefill: the weight stream sets the time.
+// FP8-blockwise expert GEMMs on row tiles of up to 64 rows and block tiles of up to 128, between
+// one-token decode and prefill: the weight stream sets the time.
 //
 // One 16x16x128 MFMA per 128-K scale block, in the arithmetic of the kernels it stands in for,
 // so h and y are the same bits: on row tiles acc += part * (s_a[row, k] * s_w[k])
@@ -29,7 +29,7 @@
 //    load: 3883 and 1211 us), the weight loads spread over the step (3210, 899), wave priority
 //    for the MFMAs (3134, 865).
 //
-// Measured where the rules of its use stand (gemm_fp8.hip launch_gemm, kMidMaxRows): DeepSeek-V3
+// Measured where the rules of its use stand (gemm_fp8.hip launch_gemm, kMidTallMaxRows): DeepSeek-V3
 // at 600 tokens 11.3 GB of weights in a layer of 1841 us, 6.1 TB/s (ring kernels 2050 us).
 //
 // Fragment layout (16x16x128): lane l supplies row l % 16 and, with g = l / 16, the bytes
@@ -245,11 +245,10 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
   const uint32_t w0_base = lds_addr(&s.sw[KIND == 0 ? 0 : wave >> 1][0]);
   const uint32_t w1_base = lds_addr(&s.sw[KIND == 0 ? 1 : wave >> 1][0]);
   const uint32_t r_base = lds_addr(s.r) + 4 * r16 + (KIND == 1 ? 4 * TR * (wave >> 1) : 0);
-  // Scale ratios: lane j of wave w owns row 64 (w % 2) + j of half w / 2 (of 64 rows: row
-  // 32 (w % 2) + j % 32, the upper lanes repeat the lower ones) and writes block k + 1's
-  // during step k. Rows without a source use scale 1; a zero scale (an all-zero weight block,
+  // Scale ratios (TR = 128): lane j of wave w owns row 64 (w % 2) + j of half w / 2 and writes
+  // block k + 1's during step k. Rows without a source use scale 1; a zero scale (an all-zero weight block,
   // whose products are zero) repeats the previous one.
-  const int orow = (TR / 2) * (wave & 1) + (lane & (TR / 2 - 1)), ohalf = wave >> 1;
+  const int orow = 64 * (wave & 1) + lane, ohalf = wave >> 1;
   const uint32_t osa = lds_addr(s.sa) + 16 * orow;
   const uint32_t osw = lds_addr(&s.sw[ohalf][0]);
   const uint32_t odst = lds_addr(s.r) + 4 * (TR * ohalf + orow);
@@ -453,10 +452,10 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
   }
 }
 
-// RATIO: the block kernels' arithmetic on block tiles; otherwise the row-tile kernels' on row
-// tiles.
-template <int KIND, int TR, bool RATIO>
+// TR = 128: the block kernels' arithmetic on block tiles; 64: the row-tile kernels' on row tiles.
+template <int KIND, int TR>
 __global__ __launch_bounds__(kMidThreads, TR > 64 ? 2 : 3) void expert_gemm_mid_kernel(MidArgs p) {
+  constexpr bool RATIO = TR > 64;
   __shared__ __attribute__((aligned(1024))) uint8_t sB[kMidCols * 128];
   __shared__ __attribute__((aligned(1024))) uint8_t sA[2 * TR * 128];
   __shared__ __attribute__((aligned(1024))) uint8_t sSA[2 * TR * 16];
@@ -519,31 +518,29 @@ bool mid_fits(int kind, const MidArgs& a) {
          2UL * a.I * a.H < lim && a.rows < (1L << 31);
 }
 
-template <int TR, bool RATIO>
+template <int TR>
 static void launch_mid_tiles(int kind, const MidArgs& a, long items, hipStream_t st) {
   const dim3 grid((unsigned)items), block(kMidThreads);
   if (kind == 0)
-    hipLaunchKernelGGL((expert_gemm_mid_kernel<0, TR, RATIO>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((expert_gemm_mid_kernel<0, TR>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((expert_gemm_mid_kernel<1, TR, RATIO>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((expert_gemm_mid_kernel<1, TR>), grid, block, 0, st, a);
 }
 
-void launch_mid(int kind, const MidArgs& a, int max_tiles, int rows, hipStream_t st) {
+void launch_mid(int kind, const MidArgs& a, int max_tiles, hipStream_t st) {
   const long NT = (kind == 0) ? a.I / 128 : a.H / kMidCols;
-  if (a.seg == nullptr) return launch_mid_tiles<kMidTileRows, false>(kind, a, (long)max_tiles * NT, st);
-  const long items = 8L * block_tiles_cap(max_tiles) * NT;  // each XCD's share of the block tiles
-  if (rows > kMidTileRows)
-    launch_mid_tiles<kMidTallRows, true>(kind, a, items, st);
-  else
-    launch_mid_tiles<kMidTileRows, true>(kind, a, items, st);
+  if (a.seg == nullptr)
+    launch_mid_tiles<kMidTileRows>(kind, a, (long)max_tiles * NT, st);
+  else  // each XCD's share of the block tiles
+    launch_mid_tiles<kMidTallRows>(kind, a, 8L * block_tiles_cap(max_tiles) * NT, st);
 }
 
 }  // namespace moe
 
 using namespace moe;
 
-int moe::mid_max_tiles(int T, int K, int E, int n_shared, int tile_rows) {
+int moe::mid_max_tiles(int T, int K, int E, int n_shared) {
   const long rows = (long)T * std::min(K, E);
-  return (int)(rows / tile_rows + std::min<long>(E, rows) +
-               (long)n_shared * ((T + tile_rows - 1) / tile_rows));
+  return (int)(rows / kMidTallRows + std::min<long>(E, rows) +
+               (long)n_shared * ((T + kMidTallRows - 1) / kMidTallRows));
 }

@@ -32,8 +32,8 @@ struct MidArgs {
 // of 512 (whole groups of four K blocks, whole column tiles) up to 16384, aligned operands,
 // and operands that 32-bit byte offsets reach. Otherwise the other kernels run.
 bool mid_fits(int kind, const MidArgs& a);
-// Launch on a.tiles: block tiles (a.seg set, XCD ranges in the header num_tiles) or row tiles,
-// of at most `rows` rows: kMidTileRows, or for block tiles kMidTallRows.
-void launch_mid(int kind, const MidArgs& a, int max_tiles, int rows, hipStream_t st);
+// Launch on a.tiles: block tiles of at most kMidTallRows rows (a.seg set, XCD ranges in the header
+// num_tiles) or row tiles of at most kMidTileRows.
+void launch_mid(int kind, const MidArgs& a, int max_tiles, hipStream_t st);
 
 }  // namespace moe

@@ -28,19 +28,20 @@ constexpr int kBlockTileRows = 256;
 // Rows per tile of the prefill-sized MXFP4 expert GEMM kernels.
 constexpr int kMxBlockTileRows = 128;
 
-// Rows per tile of the mid-size fp8 expert GEMM kernels (gemm_fp8_mid.hip). The layer runs
-// them instead of the block kernels from 32 routed rows per expert on average: 64-row tiles up
-// to kMidMaxRows, 128-row tiles up to kMidTallMaxRows.
-// Layer, block -> 64-row kernels, at 33 rows DeepSeek-V3 2127 -> 2020 us and Kimi-K2
-// 3134 -> 3051 us, at 35 GLM-4.5 805 -> 741 us; at 41 DeepSeek-V3 2165 -> 2158 us; at 50 and
-// above, where experts take two 64-row tiles, they lose (DeepSeek-V3 2241 -> 2294 us).
-// Block -> 128-row kernels: at 42 rows Kimi-K2 3228 -> 3132 and GLM-4.5 827 -> 803 us, at 75
-// DeepSeek-V3 2405 -> 2365, Kimi-K2 3613 -> 3584 and GLM-4.5 920 -> 863 us; at 81 and 83
-// DeepSeek-V3 2462 -> 2486 and Kimi-K2 3688 -> 3692 us (GLM-4.5 gains up to 115), at 125 to 256
-// the block kernels lead by up to 4 % (two thirds of the global -> LDS bytes per product).
+// Rows per tile of the mid-size fp8 expert GEMM kernels (gemm_fp8_mid.hip): row tiles, and the
+// block tiles on which the layer runs them instead of the block kernels from 32 to
+// kMidTallMaxRows routed rows per expert on average.
+// Layer, block -> mid-size kernels, us: at 34 rows Kimi-K2 3164 -> 3004 and GLM-4.5 827 -> 721,
+// at 36 DeepSeek-V3 2170 -> 2027, at 75 DeepSeek-V3 2445 -> 2331, Kimi-K2 3642 -> 3440 and GLM-4.5
+// 983 -> 865; with Zipf(1.2) routing at 34 rows Kimi-K2 2722 -> 2665 and GLM-4.5 748 -> 668, at 72
+// DeepSeek-V3 2411 -> 2327. At 81 and 83 rows DeepSeek-V3 2462 -> 2486 and Kimi-K2 3688 -> 3692
+// (GLM-4.5 gains up to 115), at 125 to 256 the block kernels lead by up to 4 % (two thirds of the
+// global -> LDS bytes per product). Block tiles of 64 rows, three workgroups per CU, were 1 to 2 %
+// faster up to 40 rows under even routing (Kimi-K2 34 rows 2950), but experts of many such
+// tiles under Zipf routing cost more than the block kernels' (Kimi-K2 34 rows 2826, DeepSeek-V3 36
+// rows 1995 against 1940), and the host does not know the routing.
 constexpr int kMidTileRows = 64;
 constexpr int kMidTallRows = 128;
-constexpr int kMidMaxRows = 40;
 constexpr int kMidTallMaxRows = 76;
 // Work items from which they run 16-row tiles (four per CU), and 32-row tiles and small layers
 // (two per CU).
@@ -171,8 +172,8 @@ int layer_down_combine_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, in
                           const int32_t* ids, const int32_t* inv, const float* weights,
                           void* out_bf16, void* stream, bool* done);
 
-// Most block tiles of tile_rows rows that the layer's mapping writes (compact rows).
-int mid_max_tiles(int T, int K, int E, int n_shared, int tile_rows);
+// Most block tiles of kMidTallRows rows that the layer's mapping writes (compact rows).
+int mid_max_tiles(int T, int K, int E, int n_shared);
 
 // Most block tiles of kMxBlockTileRows rows that the layer's mapping writes (compact rows).
 int mx_block_max_tiles(int T, int K, int E);
