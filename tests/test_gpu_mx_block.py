@@ -35,8 +35,8 @@ def _ring_experts(x, ids, wts, w, act, gl, ul, B=256):
 
 
 # T * K / E > 32 in all of them. H = I = 512: one scale group, two steps; 1536 x 1024: odd
-# numbers of groups; 768: not a multiple of 512, which stays on the row-tile kernels. The first
-# and 1025 tokens run block tiles, the others have too few items for them.
+# numbers of groups; 768: not a multiple of 512, which stays on the row-tile kernels. 1025
+# tokens run block tiles, the others have too few items for them.
 @pytest.mark.parametrize("T,E,K,H,I,act,bias,skew", [
     (67, 2, 1, 512, 512, "swish", True, [0.0, -60.0]),         # one expert holds all 67 rows, one none
     (129, 4, 2, 512, 512, "silu", False, [30.0, 0.0, 0.0, -30.0]),  # a 129-row expert: two 65-row tiles

@@ -39,8 +39,8 @@ def test_row_tiles(T, H, I, E, rows, on_block):
 # Above 32 rows per expert: block tiles of up to 128 rows, but 64-row tiles on the ring kernels
 # where one round of those holds both products (tall tiles are then longer chains of the same work).
 @pytest.mark.parametrize("T,H,I,E,K,rows", [
-    (66, 512, 512, 4, 2, 128), (80, 512, 512, 4, 2, 128),       # up to 40 rows: an expert is one tile in both
-    (84, 512, 512, 4, 2, 64), (512, 512, 512, 4, 2, 64), (600, 1024, 1024, 8, 2, 64),
+    (66, 512, 512, 4, 2, 64), (260, 512, 512, 16, 2, 64), (160, 1024, 1024, 8, 2, 64),  # 33 to 40 rows
+    (512, 512, 512, 4, 2, 64), (600, 1024, 1024, 8, 2, 64),
     (256, 3072, 3072, 4, 2, 64), (300, 3072, 3072, 4, 2, 128),  # 288 and 336 gate_up items
     (1024, 1536, 512, 16, 2, 64), (1200, 1536, 512, 16, 2, 128),  # 288 and 324 down items
     (257, 3072, 3072, 32, 4, 128), (2048, 3072, 3072, 128, 4, 128)])

@@ -450,19 +450,20 @@ static int mx_layer_rows(int T, int H, int I, int E, int K, int B, bool block_ok
   return tall ? 64 : 32;
 }
 
-// Whether the MXFP4 layer runs block tiles: above 32 rows per expert, up to 40 of them (an expert is
-// one tile of the ring kernels too), or where 64-row tiles are more than one round of the ring
-// kernels' one workgroup per CU in one product (from 320 items, counted with a remainder tile for
-// each expert). In one round a taller tile is only a longer chain. Layer, 64-row
-// tiles on the ring -> block tiles, us: 4 experts of 512 x 512 at 33 / 50 / 64 / 100 / 256 rows per
-// expert 35.8 / 36.3 / 36.9 / 37.2 / 43.3 -> 32.2 / 34.0 / 36.7 / 41.1 / 47.2; 8 of 1024 x 1024 at 40 / 80 /
-// 200 / 256 (264 and 320 items) 43.3 / 50.6 / 54.0 / 65.7 -> 40.8 / 53.3 / 54.3 / 56.9; 4 of 3072 x 3072
-// at 128 / 150 (288 and 336 items) 71.3 / 98.7 -> 80.2 / 74.5.
+// Whether the MXFP4 layer runs block tiles: above 32 rows per expert, where 64-row tiles are more
+// than one round of the ring kernels' one workgroup per CU in one product (from 320 items, counted
+// with a remainder tile for each expert). In one round a taller tile is only a longer chain. Layer,
+// 64-row tiles on the ring -> block tiles, us: 4 experts of 512 x 512 at 64 / 100 / 256 rows per
+// expert 36.9 / 37.2 / 43.3 -> 36.7 / 41.1 / 47.2; 8 of 1024 x 1024 at 80 / 200 / 256 (264 and 320
+// items) 50.6 / 54.0 / 65.7 -> 53.3 / 54.3 / 56.9; 4 of 3072 x 3072 at 128 / 150 (288 and 336 items)
+// 71.3 / 98.7 -> 80.2 / 74.5. Up to 40 rows an expert is mostly one tile in both, and block tiles gain
+// under even routing (16 of 512 x 512, 36 rows: 42.8 -> 37.6) but lose under Zipf routing (43.5 ->
+// 47.3; 8 of 1024 x 1024, 33 rows: 43.4 -> 49.4), which the host does not know.
 constexpr long kMxBlockMinItems = 320;
 static bool mx_layer_block(int T, int H, int I, int E, int K, int B) {
   if (!use_block(T, K, E)) return false;
   const long R = routed_rows(T, K, E), tiles = (R + std::min(64, B) - 1) / std::min(64, B) + E;
-  return R <= 40L * E || tiles * std::max(I / 128, H / 256) >= kMxBlockMinItems;
+  return tiles * std::max(I / 128, H / 256) >= kMxBlockMinItems;
 }
 
 extern "C" int moe_layer_mx_tile_rows(int T, int H, int I, int E, int K, int B) {
