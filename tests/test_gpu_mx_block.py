@@ -88,7 +88,7 @@ def test_layer_block_tiles_of_every_height(cuda, H, I, act, bias):
 @pytest.mark.parametrize("T,E,K,H,I,act,B,rows,on_block", [
     (160, 128, 4, 512, 512, "swish", 256, 32, 1),
     (700, 160, 4, 512, 1024, "silu", 256, 32, 3),
-    (300, 136, 4, 1024, 1024, "silu", 256, 64, 3),   # the operator path: 32 rows
+    (700, 136, 4, 1024, 1024, "silu", 256, 64, 3),   # 20 rows per expert; the operator path: 32 rows
     (1200, 160, 4, 1024, 512, "swish", 256, 64, 3),  # 30 rows per expert: 64 rows in both
     (250, 64, 4, 2560, 1536, "swish", 256, 32, 2),
     (900, 128, 4, 1024, 512, "swish", 16, 64, 3),   # 16-slot blocks: every tile at most 16 rows

@@ -29,7 +29,9 @@ def test_gpt_oss_20b_row_tiles(T, rows, on_block):
 @pytest.mark.parametrize("T,H,I,E,rows,on_block", [
     (48, 4096, 4096, 24, 32, RING),        # 768 gate_up items of K = 4096
     (108, 1024, 1024, 96, 32, GATE_UP),    # of K = 1024: the block kernel even at 768; down on the ring
-    (144, 1024, 512, 128, 64, BOTH),       # 512 and 512: one round of the block kernels
+    (144, 1024, 512, 128, 32, BOTH),       # 584 and 584 items: below 1024 of 64-row tiles, up to 16 rows
+    (96, 2048, 1024, 64, 32, BOTH), (256, 2048, 1024, 64, 32, BOTH), (272, 2048, 1024, 64, 64, BOTH),
+    (256, 2048, 1024, 128, 64, BOTH),      # 8 rows, 1152 and 1152 items of 64-row tiles
     (320, 1024, 2048, 64, 64, GATE_UP),    # 20 rows per expert: 64-row tiles, down on the ring
     (160, 3072, 3072, 128, 64, BOTH)])     # GPT-OSS-120B
 def test_row_tiles(T, H, I, E, rows, on_block):

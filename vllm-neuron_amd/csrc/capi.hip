@@ -435,18 +435,23 @@ extern "C" int moe_layer_forward_noalloc(
 static int mx_layer_rows(int T, int H, int I, int E, int K, int B, bool block_ok) {
   const int mt = choose_mt_mx(T, K, E), N = moe_num_blocks(T, K, E, B);
   if (!block_ok || mt != 32) return mt;
-  // Of 5 to 24 rows per expert, 64-row tiles keep nearly every expert in one tile: where the block
-  // kernels run both products on them, and from 9 rows where they run gate_up on them and down
-  // on neither height (64 experts of 1024 x 2048, 20 rows: 87 -> 75 us). With down on the ring
-  // kernels they lose below that (160 experts of 512 x 1024, 5 / 8 rows: 57.2 / 65.5 at 32 rows, 62.9 /
-  // 69.7 us at 64), and where the ring keeps gate_up at 32 rows (GPT-OSS-20B, 33 / 64 / 80 / 135
-  // tokens 117 / 120 / 114 / 118 at 32 rows, 125 / 127 / 128 / 130 us at 64).
+  // Of 5 to 24 rows per expert, 64-row tiles keep nearly every expert in one tile: above 16 rows
+  // where the block kernels run both products on them, or gate_up on them and down on neither
+  // height (64 experts of 1024 x 2048, 20 rows: 87 -> 75 us), below that where they have 1024 items in
+  // both, two rounds (GPT-OSS-120B under Zipf routing, 8 / 12 / 16 rows 191 / 243 / 263 -> 179 / 214 /
+  // 230 us, even routing within 1 %). In one round the tallest tile sets the time, which shows under
+  // skewed routing (64 experts of 2048 x 1024 under Zipf routing, 4 to 6 rows: 43.5 to 45.2 at 32 rows,
+  // 46.9 to 49.4 us at 64). They lose too with down on the ring kernels (160 experts of 512 x 1024, 5 /
+  // 8 rows: 57.2 / 65.5 at 32 rows, 62.9 / 69.7 us at 64), and where the ring keeps gate_up at 32 rows
+  // (GPT-OSS-20B, 33 / 64 / 80 / 135 tokens 117 / 120 / 114 / 118 at 32 rows, 125 / 127 / 128 / 130 us
+  // at 64).
   const int t32 = moe_max_tiles(T, K, E, N, B, 0, 32), t64 = moe_max_tiles(T, K, E, N, B, 0, 64);
   auto on_block = [&](int kind, int rows) {
     return mx_rows_on_block(kind, H, I, E, rows == 32 ? t32 : t64, rows);
   };
   if (!on_block(0, 32) || !on_block(0, 64)) return 32;
-  const bool tall = on_block(1, 64) || (!on_block(1, 32) && routed_rows(T, K, E) > 8L * E);
+  const bool many = routed_rows(T, K, E) > 16L * E || (long)t64 * std::min(I / 128, H / 256) >= 2 * kMidMinItems;
+  const bool tall = many && (on_block(1, 64) || !on_block(1, 32));
   return tall ? 64 : 32;
 }
 
