@@ -373,6 +373,11 @@ int moe_expert_down_mx(const uint8_t* hq, const uint8_t* hs, int T, int H, int I
  * kernels). Host only. */
 int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B);
 
+/* Which of the fp8 products run the mid-size kernels on a list of at most max_tiles row tiles of
+ * mt rows, with aligned operands: bit 0 gate_up, bit 1 down; the ring kernels run the others.
+ * Host only. */
+int moe_row_tile_kernels(int H, int I, int max_tiles, int mt);
+
 /* Which of the MXFP4 products run the block kernels on a list of at most max_tiles row tiles of
  * mt rows, with 16-byte aligned operands and no shared experts: bit 0 gate_up, bit 1 down; the
  * ring kernels run the others. Host only. */

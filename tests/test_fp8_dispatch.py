@@ -10,6 +10,22 @@ def _rows(T, H, I, E, K, S=0, B=256):
     return _lib.load().moe_layer_tile_rows(T, H, I, E, K, S, B)
 
 
+RING, GATE_UP, DOWN, BOTH = 0, 1, 2, 3
+
+
+# 16-row tiles: the mid-size kernels from 1024 items, 2048 where K is above 5120.
+@pytest.mark.parametrize("T,H,I,E,on_mid", [
+    (2, 7168, 2048, 384, RING), (4, 7168, 2048, 384, RING),      # 35 tiles: 560 gate_up and 980 down items
+    (8, 7168, 2048, 384, DOWN), (8, 7168, 2048, 256, DOWN), (14, 7168, 2048, 384, DOWN),  # 1104 to 1920 gate_up
+    (15, 7168, 2048, 384, BOTH), (64, 7168, 2048, 256, BOTH),
+    (9, 5120, 1536, 160, DOWN), (10, 5120, 1536, 160, BOTH)])    # 936 and 1044 gate_up items of K = 5120
+def test_sixteen_row_kernels(T, H, I, E, on_mid):
+    lib = _lib.load()
+    assert _rows(T, H, I, E, 8, 1) == 16
+    tiles = lib.moe_max_tiles(T, 8, E, lib.moe_num_blocks(T, 8, E, 256), 256, 1, 16)
+    assert lib.moe_row_tile_kernels(H, I, tiles, 16) == on_mid
+
+
 # 5 to 24 rows per expert: 64-row tiles only where both products have 512 items of them.
 @pytest.mark.parametrize("T,H,I,E,K,S,rows", [
     (16, 4096, 14336, 8, 2, 0, 16), (24, 4096, 14336, 8, 2, 0, 32),  # 1008 gate_up, 144 down items

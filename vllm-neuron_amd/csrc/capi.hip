@@ -175,6 +175,17 @@ static bool layer_mid(int T, int I, int E, int K, int n_shared) {
          (long)mid_max_tiles(T, K, E, n_shared) * (I / 128) >= kMidMinItems;
 }
 
+extern "C" int moe_row_tile_kernels(int H, int I, int max_tiles, int mt) {
+  if (H <= 0 || I <= 0 || max_tiles <= 0) return 0;
+  MidArgs a{};
+  a.H = H;
+  a.I = I;
+  int on_mid = 0;
+  for (int kind = 0; kind < 2; ++kind)
+    on_mid |= (mid_rows(kind, H, I, max_tiles, mt) && mid_fits(kind, a)) << kind;
+  return on_mid;
+}
+
 extern "C" int moe_layer_tile_rows(int T, int H, int I, int E, int K, int n_shared, int B) {
   if (T <= 0 || H <= 0 || I <= 0 || E <= 0 || K <= 0 || n_shared < 0 || B <= 0) return 0;
   MidArgs a{};

@@ -450,21 +450,8 @@ __global__ void selftest_mfma_kernel(const uint8_t* a, const uint8_t* b, float* 
 
 template <int KIND>
 static int launch_gemm(const GemmArgs& a, int max_tiles, int mt, hipStream_t st) {
-  // Tiles of up to 64 rows run the mid-size kernels (three workgroups per CU, the same output
-  // bits): whole layer, ring kernels -> mid-size kernels, DeepSeek-V3 at 257 / 600 / 1000
-  // tokens 1850 / 2050 / 2290 -> 1769 / 1841 / 1955 us, GLM-4.5 at 100 / 500 tokens 667 / 893
-  // -> 610 / 681 us, Kimi-K2 at 600 / 1200 tokens 2857 / 3340 -> 2660 / 2841 us. 16- and 32-row
-  // tiles only where the items fill the chip twice, or four times at 16 rows (GLM-4.5 30 tokens
-  // 503 -> 481 us, DeepSeek-V3 16 tokens 723 -> 688 us, 64 tokens 1472 -> 1427 us): below that an
-  // item is a chain of K steps, which the ring's three stages shorten (DeepSeek-V3 2 tokens, 272
-  // items: 133 against 158 us; the small layer's 32 items at 64 tokens: 36.6 against 37.5 us;
-  // with the ring from 512 to 1024 items, DeepSeek-V3 at 4 / 5 / 7 tokens 292 / 314 / 395 -> 282 /
-  // 305 / 391 us and Kimi-K2 at 5 / 6 323 / 347 -> 317 / 343, though Kimi-K2 at 4 goes 255 -> 256
-  // and GLM-4.5 at 5 180 -> 185).
-  // The ring at 64 rows (four fragments per wave and step) loses there too (small layer at
-  // 100 tokens 49 against 41 us).
-  const long items_mid = (long)max_tiles * ((KIND == 0) ? a.I / 128 : a.H / 256);
-  if (mt == 64 || (mt <= 32 && items_mid >= (mt <= 16 ? kMidMinItems16 : kMidMinItems))) {
+  // The mid-size kernels (three workgroups per CU, the same output bits) where mid_rows says so
+  if (mid_rows(KIND, a.H, a.I, max_tiles, mt)) {
     MidArgs m{};
     m.a = a.a;
     m.as = a.as;

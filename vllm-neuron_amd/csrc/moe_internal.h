@@ -43,8 +43,8 @@ constexpr int kMxBlockTileRows = 128;
 constexpr int kMidTileRows = 64;
 constexpr int kMidTallRows = 128;
 constexpr int kMidTallMaxRows = 76;
-// Work items from which they run 16-row tiles (four per CU), and 32-row tiles and small layers
-// (two per CU).
+// Work items from which they run 16-row tiles (four per CU; see mid_rows), and 32-row tiles and
+// small layers (two per CU).
 constexpr long kMidMinItems16 = 1024;
 constexpr long kMidMinItems = 512;
 

@@ -71,6 +71,7 @@ PROTOTYPES = {
     "moe_expert_down_mx": (_i, [_p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p,
                                 _i, _i, _p, _p]),
     "moe_selftest_mfma_mx": (_i, [_p, _p, _p, _p, _i, _p, _p]),
+    "moe_row_tile_kernels": (_i, [_i, _i, _i, _i]),
     "moe_layer_tile_rows": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "moe_mx_row_tile_kernels": (_i, [_i, _i, _i, _i, _i]),
     "moe_layer_mx_tile_rows": (_i, [_i, _i, _i, _i, _i, _i]),
