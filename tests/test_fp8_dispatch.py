@@ -1,9 +1,12 @@
 """Rows per tile of the fp8 layer, by sizes: host rules, no GPU needed. The results of all tile
 heights are the same bits (test_gpu_mid_tiles.py); these are the sizes where one of them was
 measured slower."""
-import pytest
+from types import SimpleNamespace
 
-from vllm_neuron_amd import _lib
+import pytest
+import torch
+
+from vllm_neuron_amd import _lib, ops
 
 
 def _rows(T, H, I, E, K, S=0, B=256):
@@ -46,3 +49,15 @@ def test_row_tiles(T, H, I, E, K, S, rows):
     (160, 1024, 512, 8, 2, 0, 256), (520, 2048, 768, 128, 8, 0, 256)])  # 10 x 4; I not a multiple of 512
 def test_block_tiles(T, H, I, E, K, S, rows):
     assert _rows(T, H, I, E, K, S) == rows
+
+
+# The operators' block tile lists are as tall as the layer's; channel scales keep 256 rows.
+@pytest.mark.parametrize("T,H,I,E,K,S,rows", [
+    (1500, 5120, 1536, 160, 8, 0, 128), (250, 5120, 1536, 40, 8, 1, 128),  # 12 x 58 items
+    (560, 2048, 1024, 48, 6, 2, 128), (400, 2048, 768, 48, 6, 2, 256), (1700, 5120, 1536, 160, 8, 0, 256)])
+def test_operators_take_the_layers_block_tiles(T, H, I, E, K, S, rows):
+    w = SimpleNamespace(hidden=H, w13=torch.empty(E, 2 * I, 0), n_shared=S, has_channel_scales=False)
+    assert ops.use_block_kernels(T, K, E)
+    assert ops.block_tile_rows(T, K, E, w) == rows == _rows(T, H, I, E, K, S)
+    w.has_channel_scales = True
+    assert ops.block_tile_rows(T, K, E, w) == 256

@@ -48,19 +48,17 @@ def num_blocks(T, K, E, B):
 
 
 def use_block_kernels(T, K, E):
-    """The layer switches to the 256x256 block kernels above 32 rows per expert on
-    average (the measured crossover against every row-tile height)."""
+    """Block tiles instead of row tiles, as the layer takes them: above 32 rows per expert on
+    average (block_tile_rows gives their height)."""
     return -(-T * min(K, E) // E) > 32
 
 
 def block_tile_rows(T, K, E, w):
-    """Rows per tile of the block tile lists for weights w: 128 (kernels with two workgroups per
-    CU) up to 76 rows per expert on average, the layer's bound, where the weights suit them
-    and fill the chip; else 256."""
+    """Rows per tile of the block tile lists for weights w: 128 where the layer runs the mid-size
+    kernels on such tiles (they take no channel scales), else 256."""
     H, I = w.hidden, w.w13.shape[1] // 2
-    tall = (T * min(K, E) <= 76 * E and H % 512 == 0 and I % 512 == 0
-            and not w.has_channel_scales and E * (I // 128) >= 512)
-    return 128 if tall else 256
+    rows = _lib.load().moe_layer_tile_rows(T, H, I, E, K, w.n_shared, 256)
+    return 128 if rows == 128 and not w.has_channel_scales else 256
 
 
 def choose_mt(T, K, E):
