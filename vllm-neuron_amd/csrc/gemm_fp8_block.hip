@@ -820,7 +820,7 @@ extern "C" int moe_max_block_tiles(int T, int K, int E, int N, int B, int n_shar
 
 extern "C" size_t moe_block_tiles_workspace_bytes(int N, int max_tiles) {
   if (N <= 0 || max_tiles <= 0) return 0;
-  return (size_t)N * 8 + (size_t)max_tiles * 24 + 256;
+  return (size_t)N * 4 + 256;  // the blocks' lengths, which more than kSegLds blocks keep here
 }
 
 static int build_block_tiles(const char* _moe_fn, const int32_t* token_position_to_id,
