@@ -116,10 +116,6 @@ __device__ __forceinline__ void lds_frag_issue(uint32_t lo_addr, uint32_t hi_add
 __device__ __forceinline__ void lds_frag_wait(v4i& lo, v4i& hi) {
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo), "+v"(hi) : : "memory");
 }
-template <int OFF>
-__device__ __forceinline__ void lds_v4_issue(uint32_t addr, v4i& v) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
-}
 __device__ __forceinline__ void lds_v4_wait(v4i& v) {
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v) : : "memory");
 }
@@ -381,10 +377,10 @@ __device__ __forceinline__ void block_item(const BlkArgs& p, const BlkLds& s, co
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
       switch (m) {
-        case 0: lds_v4_issue<0>(addr, r[m]); break;
-        case 1: lds_v4_issue<64>(addr, r[m]); break;
-        case 2: lds_v4_issue<128>(addr, r[m]); break;
-        default: lds_v4_issue<192>(addr, r[m]); break;
+        case 0: lds_read16<0>(addr, r[m]); break;
+        case 1: lds_read16<64>(addr, r[m]); break;
+        case 2: lds_read16<128>(addr, r[m]); break;
+        default: lds_read16<192>(addr, r[m]); break;
       }
     }
   };
@@ -419,7 +415,7 @@ __device__ __forceinline__ void block_item(const BlkArgs& p, const BlkLds& s, co
     float sa;
     if (sgrp) {
       if ((kb & 3) == 0) {
-        lds_v4_issue<0>(sa_own(kb), s4);
+        lds_read16<0>(sa_own(kb), s4);
         lds_v4_wait(s4);
       }
       const int k3 = kb & 3;

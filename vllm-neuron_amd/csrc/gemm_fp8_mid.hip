@@ -58,18 +58,10 @@ struct MidLds {
   float* r;           // scale ratios [step & 1][half][row]; at the end the waves' row maxima [4][row]
 };
 
-// LDS reads left in flight until a wait names their registers (in asm: the compiler would
-// wait for every direct-to-LDS load in flight before a plain read).
-template <int OFF>
-__device__ __forceinline__ void mid_read16(uint32_t addr, v4i& v) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
-}
+// LDS reads left in flight (lds_read16) until a wait names their registers.
 template <int OFF>
 __device__ __forceinline__ void mid_read4(uint32_t addr, float& v) {
   asm volatile("ds_read_b32 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
-}
-__device__ __forceinline__ void mid_st32(uint32_t addr, int v) {
-  asm volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(v) : "memory");
 }
 // A token fragment (16 rows) and the lane's token's scale ratios (gate_up: gate and up half;
 // down: the wave's half), or its scale in r0.
@@ -98,8 +90,8 @@ template <int KIND, int TR, int BUF, int Q, bool RATIO>
 __device__ __forceinline__ void mid_read_a(uint32_t lo, uint32_t hi, uint32_t r_addr, int m, MidFragA& f) {
 #define MID_A(M)                                                                \
   case M:                                                                       \
-    mid_read16<128 * TR * BUF + 2048 * M>(lo, f.lo);                            \
-    mid_read16<128 * TR * BUF + 2048 * M>(hi, f.hi);                            \
+    lds_read16<128 * TR * BUF + 2048 * M>(lo, f.lo);                            \
+    lds_read16<128 * TR * BUF + 2048 * M>(hi, f.hi);                            \
     if constexpr (RATIO) {                                                      \
       mid_read4<8 * TR * BUF + 64 * M>(r_addr, f.r0);                           \
       mid_read4<8 * TR * BUF + 64 * M + (KIND == 0 ? 4 * TR : 0)>(r_addr, f.r1); \
@@ -109,13 +101,6 @@ __device__ __forceinline__ void mid_read_a(uint32_t lo, uint32_t hi, uint32_t r_
     break;
   switch (m) { MID_A(0) MID_A(1) MID_A(2) MID_A(3) MID_A(4) MID_A(5) MID_A(6) MID_A(7) }
 #undef MID_A
-}
-
-// Keeps four accumulators' MFMAs before this point (nothing is read): the compiler otherwise
-// delays them past the next fragments' reads and runs out of registers. Placed one
-// fragment behind, so no MFMA result is still on its way.
-__device__ __forceinline__ void mid_pin(v4f (&c)[4]) {
-  asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]));
 }
 
 __device__ __forceinline__ v8i mid_cat(const v4i& lo, const v4i& hi) {
@@ -221,13 +206,13 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
   for (int i = 0; i < NA; ++i) load_a(i, 0, 0);
   if (wave < TR / 64) {
     load_s(0);
-    mid_st32(lds_addr(s.tok) + 4 * srow, ssrc);
+    lds_st32(lds_addr(s.tok) + 4 * srow, ssrc);
   }
   // weight block scales of the tile's two 128-row halves (gate / up, or two output blocks)
   for (int i = tid; i < 2 * KB; i += kMidThreads) {
     const int h = i < KB ? 0 : 1, kb = i - h * KB;
     const int rb = (KIND == 0) ? (h == 0 ? nt : p.I / 128 + nt) : nt * 2 + h;
-    mid_st32(lds_addr(&s.sw[h][kb]), __float_as_int(wsb[(size_t)rb * KB + kb]));
+    lds_st32(lds_addr(&s.sw[h][kb]), __float_as_int(wsb[(size_t)rb * KB + kb]));
   }
 
   v4f acc[MF][4];
@@ -272,14 +257,14 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
     float nsa, nsw;
     MidFragA f[D];
     constexpr int r1 = 16, r2 = KIND == 0 ? 128 : 32, r3 = KIND == 0 ? 144 : 48;
-    mid_read16<0>(b_lo, b[0]);
-    mid_read16<0>(b_hi, b[1]);
-    mid_read16<r1 * 128>(b_lo, b[2]);
-    mid_read16<r1 * 128>(b_hi, b[3]);
-    mid_read16<r2 * 128>(b_lo, b[4]);
-    mid_read16<r2 * 128>(b_hi, b[5]);
-    mid_read16<r3 * 128>(b_lo, b[6]);
-    mid_read16<r3 * 128>(b_hi, b[7]);
+    lds_read16<0>(b_lo, b[0]);
+    lds_read16<0>(b_hi, b[1]);
+    lds_read16<r1 * 128>(b_lo, b[2]);
+    lds_read16<r1 * 128>(b_hi, b[3]);
+    lds_read16<r2 * 128>(b_lo, b[4]);
+    lds_read16<r2 * 128>(b_hi, b[5]);
+    lds_read16<r3 * 128>(b_lo, b[6]);
+    lds_read16<r3 * 128>(b_hi, b[7]);
     // ratios: the next block's scales (past the last block: not used); otherwise this block's
     // weight scales of the wave's gate and up (or output) half
     if constexpr (RATIO) {
@@ -298,7 +283,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
       for (int i = 0; i < NA; ++i) load_a(i, kb + 1, BUF ^ 1);
       load_b(kb + 1);
       if (Q == 0 && wave < TR / 64) load_s(grp + 1);  // past the last group: not used
-      if constexpr (RATIO) mid_st32(odst + 8 * TR * (BUF ^ 1), __float_as_int(ratio(nsa, nsw)));
+      if constexpr (RATIO) lds_st32(odst + 8 * TR * (BUF ^ 1), __float_as_int(ratio(nsa, nsw)));
     }
     if (D > 2 && MF > 1) mid_read_a<KIND, TR, BUF, Q, RATIO>(a_lo, a_hi, ra0, 1, f[1]);
     mid_wait<RATIO, (D > 2 && MF > 1) ? 4 : 0>(f[0]);
@@ -315,7 +300,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
           part[n] = mid_mfma(mid_cat(b[2 * n], b[2 * n + 1]), t, (v4f){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[m][n] += part[n] * ((KIND == 0 && n >= 2) ? c1 : c0);
-        mid_pin(acc[m]);
+        acc_pin(acc[m]);
         if (m + 1 < MF) mid_wait<RATIO>(f[(m + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -332,7 +317,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
         acc[m][n] = mid_mfma(mid_cat(b[2 * n], b[2 * n + 1]), t, acc[m][n] * ((KIND == 0 && n >= 2) ? x.r1 : x.r0));
         __builtin_amdgcn_sched_barrier(0);
       }
-      mid_pin(acc[m > 0 ? m - 1 : MF - 1]);
+      acc_pin(acc[m > 0 ? m - 1 : MF - 1]);
       if (m + 1 < MF) {
         if (D > 2 && m + 2 < MF)
           mid_wait<RATIO, 4>(f[(m + 1) % D]);
@@ -353,7 +338,7 @@ __device__ __forceinline__ void mid_item(const MidArgs& p, const MidLds& s, cons
                  : "v"(osa), "v"(osw), "v"(lds_addr(s.tok) + 4 * orow)
                  : "memory");
     ovalid = valid >= 0;
-    mid_st32(odst, __float_as_int(ratio(fsa, fsw)));
+    lds_st32(odst, __float_as_int(ratio(fsa, fsw)));
   }
   for (int grp = 0; grp < KB / 4; ++grp) {
     step(grp, std::integral_constant<int, 0>{}, true);

@@ -53,16 +53,7 @@ struct MbLds {
   int* tok;        // token (gate_up) or h row (down) of each tile row; -1: none
 };
 
-// LDS reads left in flight until a wait names their registers (LDS reads complete in
-// order). In asm, because the compiler would wait for every direct-to-LDS load in flight
-// before a plain read.
-__device__ __forceinline__ void lds_st32(uint32_t addr, int v) {
-  asm volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(v) : "memory");
-}
-template <int OFF>
-__device__ __forceinline__ void mb_read16(uint32_t addr, v4i& v) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
-}
+// LDS reads left in flight (lds_read16) until a wait names their registers.
 template <int OFF>
 __device__ __forceinline__ void mb_read1(uint32_t addr, int& v) {
   asm volatile("ds_read_u8 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
@@ -86,13 +77,6 @@ __device__ __forceinline__ void mb_wait8(v4i (&b)[8], int (&s)[8]) {
                : "memory");
 }
 
-// Keeps four accumulators' MFMAs before this point (nothing is read): the compiler
-// otherwise delays MFMAs past the reads of the next fragments, whose registers then pile
-// up. Placed one fragment behind, so no MFMA result is still on its way.
-__device__ __forceinline__ void mb_pin(v4f (&c)[4]) {
-  asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]));
-}
-
 // Weight fragment 4 h + n: column tile n, half h of the step, and its scale byte (ODD: the
 // step is the second of its scale group). Column tile n's first tile row, past the
 // wave's first: gate_up holds two gate tiles, then the two up tiles of the same columns.
@@ -101,7 +85,7 @@ __device__ __forceinline__ void mb_read_b(uint32_t b_h0, uint32_t b_h1, uint32_t
                                           int (&s)[8]) {
   constexpr int r1 = 16, r2 = KIND == 0 ? 128 : 32, r3 = KIND == 0 ? 144 : 48;
 #define MB_B(H, N, R)                                  \
-  mb_read16<(R) * 128>(H ? b_h1 : b_h0, b[4 * H + N]); \
+  lds_read16<(R) * 128>(H ? b_h1 : b_h0, b[4 * H + N]); \
   mb_read1<(R) * 16 + 8 * ODD + 4 * H>(s_addr, s[4 * H + N]);
   MB_B(0, 0, 0) MB_B(0, 1, r1) MB_B(0, 2, r2) MB_B(0, 3, r3)
   MB_B(1, 0, 0) MB_B(1, 1, r1) MB_B(1, 2, r2) MB_B(1, 3, r3)
@@ -112,8 +96,8 @@ template <int H, int ODD>
 __device__ __forceinline__ void mb_read_a(uint32_t lo, uint32_t hi, uint32_t s_addr, int m, MbFragA& f) {
 #define MB_A(M)                                    \
   case M:                                          \
-    mb_read16<kMbHalfA * H + 2048 * M>(lo, f.lo);  \
-    mb_read16<kMbHalfA * H + 2048 * M>(hi, f.hi);  \
+    lds_read16<kMbHalfA * H + 2048 * M>(lo, f.lo);  \
+    lds_read16<kMbHalfA * H + 2048 * M>(hi, f.hi);  \
     mb_read1<8 * ODD + 4 * H + 256 * M>(s_addr, f.s); \
     break;
   switch (m) {
@@ -289,7 +273,7 @@ __device__ __forceinline__ void mx_block_item(const MxArgs& p, const MbLds& s, c
             }
           }
         }
-        mb_pin(acc[m > 0 ? m - 1 : MF - 1]);
+        acc_pin(acc[m > 0 ? m - 1 : MF - 1]);
         if (m + 1 < MF) {
           if (m + 2 < MF)
             mb_wait<3>(f[(m + 1) % 3]);

@@ -162,6 +162,23 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(lds_cptr)p;
 }
 
+// An LDS read left in flight until a wait names its registers (LDS reads complete in order), and a
+// write. In asm: the compiler would wait for every direct-to-LDS load in flight before a plain one.
+template <int OFF>
+__device__ __forceinline__ void lds_read16(uint32_t addr, v4i& v) {
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF) : "memory");
+}
+__device__ __forceinline__ void lds_st32(uint32_t addr, int v) {
+  asm volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
+
+// Keeps four accumulators' MFMAs before this point (nothing is read): the compiler otherwise delays
+// them past the reads of the next fragments, whose registers then pile up. Placed one fragment
+// behind, so no MFMA result is still on its way.
+__device__ __forceinline__ void acc_pin(v4f (&c)[4]) {
+  asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]));
+}
+
 // Logical 16-byte chunk c of row r lives at chunk c ^ ((r >> 1) & 7): any 16
 // consecutive rows read at one logical chunk touch 16 distinct 16-byte bank
 // groups of the 64-bank LDS (two 128-byte rows span the banks once).
