@@ -53,7 +53,7 @@ def test_block_tiles(T, H, I, E, K, S, rows):
 
 # The operators' block tile lists are as tall as the layer's; channel scales keep 256 rows.
 @pytest.mark.parametrize("T,H,I,E,K,S,rows", [
-    (1500, 5120, 1536, 160, 8, 0, 128), (250, 5120, 1536, 40, 8, 1, 128),  # 12 x 58 items
+    (1500, 5120, 1536, 160, 8, 0, 128), (250, 5120, 1536, 40, 8, 1, 128),  # 57 tiles, 684 items
     (560, 2048, 1024, 48, 6, 2, 128), (400, 2048, 768, 48, 6, 2, 256), (1700, 5120, 1536, 160, 8, 0, 256)])
 def test_operators_take_the_layers_block_tiles(T, H, I, E, K, S, rows):
     w = SimpleNamespace(hidden=H, w13=torch.empty(E, 2 * I, 0), n_shared=S, has_channel_scales=False)

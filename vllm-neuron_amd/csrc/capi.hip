@@ -25,9 +25,9 @@ void set_error(const char* fn, const char* fmt, ...) {
 
 void clear_error() { g_err[0] = 0; }
 
-// Rows per expert tile (see use_block for the measurements): 16-row tiles up to 4
-// routed rows per expert on average, 32 up to 24, 64 up to 48 (the MX layer, which
-// has no block kernels, past 32), else 128.
+// Rows per row tile (see use_block for the measurements): 16 up to 4 routed rows per expert on
+// average, 32 up to 24 (layer_rows and mx_layer_rows raise some of them to 64), 64 up to 48, else
+// 128. Above 32 rows the fp8 layer runs block tiles, the MX layer where it has items for them.
 static int choose_mt(int T, int K, int E) {
   long avg = ((long)T * std::min(K, E) + E - 1) / E;
   if (avg <= 4) return 16;
@@ -66,13 +66,14 @@ struct LayerWs {
   size_t bytes;
 };
 
-// The 256x256 ("block") kernels take over above 32 rows per expert on average.
-// Expert GEMM time (gate_up + down) on the DeepSeek-V3 layer by rows per expert,
-// ms, row tiles of 16 / 32 / 64 rows against the block kernels: 4 rows 1.81 /
-// 1.81 / 1.93 vs 2.05; 8: 1.95 / 1.92 / 2.08 vs 2.15; 16: 2.30 / 2.03 / 2.13 vs
-// 2.29; 24: 2.78 / 2.11 / 2.19 vs 2.37; 32: 3.32 / 2.36 / 2.28 vs 2.42; 48: - /
-// 2.95 / 2.47 vs 2.51; 64: - / 3.58 / 3.01 vs 2.60. On the Kimi-K2 layer at 42.7
-// rows the block kernels lead (whole layer 3.90 against 3.95-4.00 ms), hence 32.
+// Block tiles (of whole experts, in XCD ranges) take over from row tiles above 32 rows per expert on
+// average: on the mid-size kernels up to kMidTallMaxRows, else on the 256x256 block kernels.
+// Expert GEMM time (gate_up + down) on the DeepSeek-V3 layer by rows per expert, ms, ring kernels
+// on row tiles of 16 / 32 / 64 rows against the block kernels: 4 rows 1.81 / 1.81 / 1.93 vs 2.05; 8:
+// 1.95 / 1.92 / 2.08 vs 2.15; 16: 2.30 / 2.03 / 2.13 vs 2.29; 24: 2.78 / 2.11 / 2.19 vs 2.37; 32:
+// 3.32 / 2.36 / 2.28 vs 2.42; 48: - / 2.95 / 2.47 vs 2.51; 64: - / 3.58 / 3.01 vs 2.60. On the Kimi-K2
+// layer at 42.7 rows the block kernels led (3.90 against 3.95-4.00 ms), hence 32. The
+// figures predate the mid-size kernels, which now run most of these tiles on both sides of the line.
 static bool use_block(int T, int K, int E) {
   return ((long)T * std::min(K, E) + E - 1) / E > 32;
 }

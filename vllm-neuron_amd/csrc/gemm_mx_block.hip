@@ -1,7 +1,8 @@
-// Prefill-sized MXFP4 expert GEMMs (GPT-OSS), for the layer above 32 routed rows per
-// expert. Same products, epilogue arithmetic and K order as the row-tile kernel
-// (gemm_mx.hip), on tiles tall enough that the matrix cores, not the weight stream of
-// one 64-row tile, set the time.
+// MXFP4 expert GEMMs (GPT-OSS) on block tiles of up to 128 rows (the layer above 32 routed rows per
+// expert, mx_layer_block) and on row tiles of 32 and 64 rows with enough items (the layer and the
+// operators from 5 rows per expert, mx_rows_on_block). Same products, epilogue arithmetic and K
+// order as the ring kernel (gemm_mx.hip), with two workgroups per CU, and block tiles tall enough
+// that the matrix cores, not the weight stream of one 64-row tile, set the time.
 //
 //  * A workgroup of 4 waves computes up to 128 rows x 256 weight rows (gate_up: 128
 //    gate rows + the matching 128 up rows; down: 256 outputs). A wave owns every row and
@@ -24,11 +25,11 @@
 //  * The scale bytes of 512 K values (16 per row) arrive with one 16-byte load per row
 //    every second step.
 //
-// Measured, GPT-OSS-120B (kernel trace), against the row-tile kernels' 64-row tiles: gate_up
-// 1408 -> 758 us and down 629 -> 386 us at 8192 tokens (256 rows per expert), 516 -> 292 and
-// 240 -> 157 us at 2048. Without the in-loop loads 500 us at 8192, without the MFMAs 580
-// us (1.24 TFLOP, MFMA alone 280 us): both halves and their overlap; at 2048 the weight
-// stream, 4.5 TB/s of it.
+// Measured, GPT-OSS-120B (kernel trace), against the ring kernels' 64-row tiles: gate_up 1408 -> 720
+// us and down 629 -> 380 us at 8192 tokens (256 rows per expert), 516 -> 295 and 240 -> 157 us at 2048.
+// At 8192 the MFMA pipes are busy 52 and 46 % of the time; gate_up without the in-loop loads takes
+// 500 us, without the MFMAs 580 us (1.24 TFLOP, MFMA alone 280 us): both halves and their overlap. At
+// 2048 26 and 23 %, with the weights read at 4.4 and 4.1 TB/s.
 //
 // Fragment layout as in gemm_mx.hip: lane l supplies row l % 16; with g = l / 16, the
 // fp8 K values [16 g, +16) and [64 + 16 g, +16), the fp4 K values [32 g, +32) and the
