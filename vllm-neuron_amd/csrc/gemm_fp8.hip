@@ -452,28 +452,9 @@ template <int KIND>
 static int launch_gemm(const GemmArgs& a, int max_tiles, int mt, hipStream_t st) {
   // The mid-size kernels (three workgroups per CU, the same output bits) where mid_rows says so
   if (mid_rows(KIND, a.H, a.I, max_tiles, mt)) {
-    MidArgs m{};
-    m.a = a.a;
-    m.as = a.as;
-    m.w = a.w;
-    m.ws = a.ws;
-    m.wsh = a.wsh;
-    m.wssh = a.wssh;
-    m.tpid = a.tpid;
-    m.tiles = a.tiles;
-    m.num_tiles = a.num_tiles;
-    m.hq = a.hq;
-    m.hs = a.hs;
-    m.y = a.y;
+    MidArgs m = mid_args(a);
     m.cs = a.cs;
     m.cssh = a.cssh;
-    m.T = a.T;
-    m.H = a.H;
-    m.I = a.I;
-    m.E = a.E;
-    m.nsh = a.nsh;
-    m.NB = a.NB;
-    m.rows = a.NB + (long)a.nsh * a.T;
     if (mid_fits(KIND, m)) {
       launch_mid(KIND, m, max_tiles, st);
       return MOE_OK;

@@ -861,27 +861,8 @@ extern "C" int moe_build_block_tiles_rows(const int32_t* token_position_to_id,
 // no per-channel scales); this file's kernels take any tile.
 template <int KIND>
 static void launch_block_rows(const BlkArgs& a, int tile_rows, int max_tiles, hipStream_t st) {
-  MidArgs m{};
-  m.a = a.a;
-  m.as = a.as;
-  m.w = a.w;
-  m.ws = a.ws;
-  m.wsh = a.wsh;
-  m.wssh = a.wssh;
-  m.tpid = a.tpid;
-  m.tiles = a.tiles;
+  MidArgs m = mid_args(a);
   m.seg = a.seg;
-  m.num_tiles = a.num_tiles;
-  m.hq = a.hq;
-  m.hs = a.hs;
-  m.y = a.y;
-  m.T = a.T;
-  m.H = a.H;
-  m.I = a.I;
-  m.E = a.E;
-  m.nsh = a.nsh;
-  m.NB = a.NB;
-  m.rows = a.NB + (long)a.nsh * a.T;
   if (tile_rows == kMidTallRows && a.cs == nullptr && a.cssh == nullptr && mid_fits(KIND, m))
     launch_mid(KIND, m, max_tiles, st);
   else

@@ -28,6 +28,32 @@ struct MidArgs {
   long rows;  // rows of h
 };
 
+// The operands that the ring and block kernels' arguments name alike.
+template <class A>
+MidArgs mid_args(const A& a) {
+  MidArgs m{};
+  m.a = a.a;
+  m.as = a.as;
+  m.w = a.w;
+  m.ws = a.ws;
+  m.wsh = a.wsh;
+  m.wssh = a.wssh;
+  m.tpid = a.tpid;
+  m.tiles = a.tiles;
+  m.num_tiles = a.num_tiles;
+  m.hq = a.hq;
+  m.hs = a.hs;
+  m.y = a.y;
+  m.T = a.T;
+  m.H = a.H;
+  m.I = a.I;
+  m.E = a.E;
+  m.nsh = a.nsh;
+  m.NB = a.NB;
+  m.rows = a.NB + (long)a.nsh * a.T;
+  return m;
+}
+
 // Whether the sizes and operands suit the kernels (kind 0 gate_up, 1 down): H and I multiples
 // of 512 (whole groups of four K blocks, whole column tiles) up to 16384, aligned operands,
 // and operands that 32-bit byte offsets reach. Otherwise the other kernels run.
